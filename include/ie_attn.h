@@ -136,8 +136,8 @@ hipError_t ie_fused_rope_kv_decode(const ie_bf16* q, int64_t q_stride_b, int64_t
  * heads on the current device, whatever the GQA ratio: the arrival counts (one uint32 per
  * sequence and query head, the most any ratio uses, with room for max(batch, 1024) sequences of
  * max(num_q_heads, 128) heads, padded to 256 bytes), then fp32 split-K partials, head_dim + 2
- * values per (query head, work entry), where the work entries are at most
- * ie_decode_attention_grid(batch, cdiv(num_q_heads, 2)). The arrival counts must be zero when a
+ * values per (query head, work entry), where the work entries are at most the larger of
+ * ie_decode_attention_grid(batch, units) for units = cdiv(num_q_heads, 2) and min(8, that). The arrival counts must be zero when a
  * workspace is first used (allocate it zeroed); every call that completes leaves them zero
  * again, so one workspace (of the largest size any of them needs) serves any number of calls in
  * stream order of any batch up to 1024 and any num_q_heads up to 128 (they share one count
@@ -155,18 +155,19 @@ size_t ie_decode_attention_workspace_size(int32_t batch, int32_t num_q_heads, in
  */
 size_t ie_decode_attention_workspace_counts_bytes(int32_t batch, int32_t num_q_heads);
 
-/* Upper bound on splits per sequence on the current device: the largest per-unit workgroup
- * target of any launch shape (CUs * 8 / num_units, 2-wave workgroups). A unit is a KV head and
- * one pair of its query heads: num_units = num_kv_heads * cdiv(num_q_heads / num_kv_heads, 2),
- * num_kv_heads itself at GQA ratio 2. */
+/* The largest per-unit workgroup target of any launch shape (CUs * 8 / num_units, one-wave
+ * workgroups): an upper bound on splits per sequence at GQA ratios 1 and 2. A unit of a work list
+ * is a KV head and one pair of its query heads: num_units = num_kv_heads *
+ * cdiv(num_q_heads / num_kv_heads, 2), num_kv_heads itself at ratios 1 and 2. Launches above
+ * ratio 2 cut their entries per KV head and read no list (see ie_decode_attention_planned). */
 int32_t ie_decode_attention_max_splits(int32_t num_units);
 
 /*
  * The per-unit workgroup target of the work split (qwen3-1.7b/kernels.py:20-37 TARGET) that
- * ie_decode_attention uses for `batch` sequences on the current device (num_units as above). The
- * launch fills the CUs with 16 waves each, as 8-wave workgroups (target CUs * 2 / num_units)
- * while the batch fits that target, else as 4-wave (CUs * 4 / num_units) or 2-wave (CUs * 8 /
- * num_units) workgroups, the first whose target holds the batch (the 2-wave one above that).
+ * a work list uses for `batch` sequences on the current device (num_units as above). A launch
+ * fills the CUs with 8 waves each, as 4-wave workgroups (target CUs * 2 / num_units)
+ * while the batch fits that target, else as 2-wave (CUs * 4 / num_units) or one-wave (CUs * 8 /
+ * num_units) workgroups, the first whose target holds the batch (the one-wave one above that).
  */
 int32_t ie_decode_attention_target(int32_t batch, int32_t num_units);
 
@@ -174,8 +175,7 @@ int32_t ie_decode_attention_target(int32_t batch, int32_t num_units);
  * Split-K GQA decode attention over the int8 cache, with the partial-softmax reduce folded into
  * the same launch (the sequence's last piece to finish merges its pieces). Any GQA ratio
  * num_q_heads / num_kv_heads of 1 to 16 (the reference's q-group padding, kernels.py:118-135),
- * head_dim 128; a workgroup serves one pair of a KV head's query heads, so ratios above 2 read
- * each KV row once per pair.
+ * head_dim 128; a workgroup serves all query heads of a KV head: each KV row is read once.
  * Replaces qwen3-1.7b/kernels.py:272-361 `decode_attention(q, kv_cache, cached_lens, slot_ids,
  * num_decoding, scale, out)` (kernels kernels.py:73-213 and 216-264, work split 20-70).
  *
@@ -242,7 +242,7 @@ hipError_t ie_decode_attention_noalloc(const ie_bf16* q, int64_t q_stride_b, int
  * The decode launch's work list, for tests and diagnostics: the work split of
  * qwen3-1.7b/kernels.py:20-70 (`compute_piece`, `assign_work`) as the decode kernel computes it
  * on the device. ie_decode_attention_grid(batch, num_units) is the number of work entries
- * (the decode launch's workgroups per unit: KV head x query-head pair, as above); ie_decode_attention_plan writes, for each entry
+ * (per unit: KV head x query-head pair, as above); ie_decode_attention_plan writes, for each entry
  * w, rows[4w .. 4w+3] = (sequence b, split index, splits of b, piece size in tokens), with
  * splits = 0 for an entry that has no work. rows: int32 [grid, 4] device memory.
  */
@@ -273,7 +273,8 @@ hipError_t ie_decode_step_prologue(const int32_t* cached_lens, const int32_t* nu
  * ie_decode_attention_plan wrote for the same cached_lens and num_decoding values, batch,
  * num_units (KV heads x query-head pairs) and device, 16-byte aligned, and plan_rows, their
  * count (at least ie_decode_attention_grid(batch, num_units)). Each workgroup reads its entry in
- * one load instead of deriving the work split from cached_lens. For engines that run every
+ * one load instead of deriving the work split from cached_lens (GQA ratios 1 and 2; launches above
+ * cut other entries and derive them from cached_lens all the same). For engines that run every
  * layer of a decode step over one step's metadata: compute the plan once per step. A plan that
  * does not match the arguments is undefined behaviour (its rows name the sequences, pieces and
  * merges of each workgroup).

@@ -9,60 +9,62 @@
 // launch is graph-capturable, and each workgroup finds its (sequence, piece) on the device from
 // cached_lens.
 //
-// One workgroup = 8 waves = one (sequence, piece, kv head), i.e. both query heads of the GQA
-// pair. Lane (g, c) of a wave (g = lane / 8, c = lane % 8) owns channels [16c, 16c+16) of the
-// four tokens 4g..4g+3 of the wave's 32-token block: each K and V row (128 int8) is read by 8
-// lanes with 16-byte loads, so one load instruction of a wave covers 8 full 128-byte rows.
+// One workgroup = W waves = one (sequence, piece, KV head) and all query heads of that KV head
+// (GQA ratio 1 to 16), so every cached byte is read once whatever the ratio. What bounds it is the
+// stream of int8 rows from HBM; the heads are the 16 columns of the MFMA tiles, so one head costs
+// what 16 do.
 //
-// Arithmetic (all VALU, no MFMA: the op is HBM-bound):
-//   int8 -> fp16 by byte permute into the fp16 pattern 0x64xx (= 1024 + byte) after flipping
-//   the sign bit, i.e. the fp16 value 1152 + x exactly; the 1152 offset is removed once per
-//   score (q . 1152 = 1152 * sum(q)) and once per output (sum of P).
-//   q is scaled by a power of two per head so it is exact in fp16; QK^T and PV use the
-//   fp32-accumulating v_dot2_f32_f16. QK partial dots are reduced across the 8 lanes of a row
-//   with DPP. Online softmax in base 2 per lane group; groups and waves are merged at the end
-//   (log-sum-exp), then either the output is written (one piece) or fp32 partials (m, l, acc)
-//   go to the workspace and the sequence's last piece to finish merges them (the reference's
-//   combine kernel, kernels.py:216-264, folded into the same launch).
+// The stream goes global -> LDS without registers (buffer_load ... lds, 16 bytes per lane): each
+// wave owns two stages of 32 tokens (K 4 KB, V 4 KB, scales 256 B), block j + 2 is requested as
+// soon as block j's reads are done, and no barrier runs in the loop. Eight waves per CU keep up to
+// 132 KB in flight. A lane may fetch its 16 bytes from any address but they land at consecutive
+// LDS places, so K's bank spreading (16-byte chunk c of token t at place c ^ (t & 7)) is done in
+// the global addresses; every group of 8 lanes still reads one whole 128-byte row.
+//
+// Per block and wave, v_mfma_f32_16x16x32_f16:
+//   S (32 tokens x 16 heads) = K . Q^T   A = K rows (lane (r, g): token r, channels 16 g ... and
+//                                        64 + 16 g ...), B = Q^T, 8 MFMAs
+//   online softmax in base 2             a lane holds head r's scores of 8 tokens
+//   O^T (128 channels x 16 heads) += V^T . P^T   A: lane (r, g) holds channels 8 r ... 8 r + 7 of
+//                                        the 8 tokens whose P it holds (bytes of 8 rows paired by
+//                                        permutes), B = P straight from the score registers, 8 MFMAs
+// int8 -> fp16 by byte permute into the fp16 pattern 0x64xx (= 1024 + byte) after flipping the
+// sign bit, i.e. 1152 + x, then -1152: exact. q is scaled by a power of two per head so that it
+// is exact in fp16; P * v_scale goes to fp16 under a wave-wide power of two chosen from the V
+// scales. The waves are merged at the end (log-sum-exp through LDS), then either the output is
+// written (one piece) or fp32 partials (m, l, acc) go to the workspace and the sequence's last
+// piece to finish merges them (the reference's combine kernel, kernels.py:216-264, folded into
+// the same launch).
+//
+// Measured in graphs of 20 calls of the fused form, cache streamed from HBM, against a kernel
+// that loaded rows into registers and took one query-head pair per workgroup with dot products:
+// 16/8 heads B=1 ctx 128 11.8 -> 7.2 us, B=8 ctx 512-1024 14.6 -> 10.0, B=16 ctx 4096 29.7 -> 27.3,
+// B=32 ctx 128-4096 33.4 -> 31.1 (4.7 TB/s), B=64 ctx 4096 86.7 -> 86.0 (6.45 TB/s: the stream),
+// B=256 ctx 1024 91.2 -> 91.6; 32/8 B=32 ctx 128-4096 61.9 -> 32.7, 40/8 84.5 -> 32.8, 64/4
+// 99.6 -> 22.7, 64/8 B=12 ctx 5001-8190 95.8 -> 34.7.
 #include <mutex>
 
 #include "ie_common.h"
 #include "kv_math.h"
 
-// Launch shape: 16 waves per CU (the 128-register budget allows 4 waves per SIMD), as 8-wave
-// workgroups, 2 per CU, while the batch fits their per-head target, else 4-wave workgroups
-// (4 per CU) or 2-wave workgroups (8 per CU), whose targets are twice and four times as large
-// (decode_waves). Measured on MI355X: 8 waves are best up to B = 64 (one 4096-token piece per
-// row at B=64 ctx=4096); above, the smaller workgroups keep every sequence in one resident
-// round of fitted pieces instead of the reference rule's target + B pieces: B=96 ctx=1024
-// -15 % (4 waves), B=256 ctx=512 -31 % and ctx=1024 -11 % (2 waves), long contexts level.
+// Launch shape: 8 waves per CU (what the stages leave room for in LDS), as 4-wave workgroups, 2
+// per CU, while the batch fits their per-head target, else 2-wave (4 per CU) or one-wave
+// workgroups (8 per CU), whose targets are twice and four times as large (decode_waves): every
+// sequence keeps a fitted piece in one resident round (B=256 ctx=1024, 16/8 heads: one-wave
+// workgroups 91.6 us against 121.6 for 2-wave ones, whose 384 entries per head take two rounds).
 
 namespace ie {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-// K/V/scale loads carry the non-temporal cache policy (aux bit 1, "nt" on gfx94x/gfx950): every
-// byte is read once, and streaming it past the caches raised read bandwidth from ~6.0 to
-// ~7.0 TB/s in isolation.
-#ifndef IE_DECODE_HEAD_FAST_MIN_BATCH
-#define IE_DECODE_HEAD_FAST_MIN_BATCH 0
-#endif
-#ifndef IE_DECODE_LOAD_AUX
-#define IE_DECODE_LOAD_AUX 2
-#endif
-
-constexpr int DA_WAVES_PER_CU = 16;
-constexpr int DA_U = 4;                // tokens per lane group per block
-constexpr int DA_TOK_WAVE = 8 * DA_U;  // 32 tokens per wave block
+constexpr int DA_WAVES_PER_CU = 8;
 constexpr int DA_MIN_PIECE = 128;
 constexpr int DA_MAX_SPLITS = 1024;  // per-KV-head workgroup target, at most
 constexpr int DA_D = 128;
 constexpr uint32_t K64 = 0x64646464u;
-constexpr float OFFSET = 1152.0f;  // fp16(0x64xx) = 1024 + byte, byte = x + 128
 
-
-// Workgroup target per unit (KV head x query-head pair; the KV head at GQA 2) of workgroups of
-// `waves` waves: one resident round.
+// Workgroup target per unit (a KV head in a launch; see decode_units for work lists) of workgroups
+// of `waves` waves: one resident round.
 int decode_target(int units, int waves) {
     return std::min(DA_MAX_SPLITS, std::max(1, device_cu_count() * (DA_WAVES_PER_CU / waves) /
                                                    std::max(1, units)));
@@ -70,11 +72,13 @@ int decode_target(int units, int waves) {
 // Waves per workgroup for a batch: the largest workgroup whose target holds the batch, else
 // the smallest.
 int decode_waves(int batch, int units) {
-    for (int w = 8; w > 2; w /= 2)
+    for (int w = 4; w > 1; w /= 2)
         if (batch <= decode_target(units, w)) return w;
-    return 2;
+    return 1;
 }
-// Units of a launch: KV heads x query-head pairs per KV head.
+// Units a work list is made for: KV heads x query-head pairs per KV head, the KV heads at ratios
+// 1 and 2. Launches of those ratios run from such a list; above ratio 2 a launch cuts its entries
+// per KV head (call_layout) and derives them itself.
 int decode_units(int hq, int hkv) { return hkv * ((hq / std::max(1, hkv) + 1) / 2); }
 
 
@@ -143,15 +147,7 @@ __device__ Work decode_assign(const int32_t* __restrict__ cached_lens, int nd, i
 }
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
-// The lane's index in its wave, from the lane-count instructions: with the wave index (uniform)
-// it rebuilds the thread index after the block loop, so that no register holds it there.
-__device__ __forceinline__ int lane_id() {
-    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-}
 __device__ __forceinline__ half2_t as_h2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
-__device__ __forceinline__ float fdot2(half2_t a, half2_t b, float c) {
-    return __builtin_amdgcn_fdot2(a, b, c, false);
-}
 __device__ __forceinline__ float exp2_safe(float x) { return __builtin_amdgcn_exp2f(x); }
 
 struct DecodeArgs {
@@ -172,11 +168,9 @@ struct DecodeArgs {
     // needed, piece) of workgroup index w), or null: every workgroup derives its entry itself.
     const int32_t* plan;
     int target, nwork, hq, hkv;
-    int ratio;   // query heads per KV head (GQA ratio, 1 ... 16)
-    int npairs;  // query-head pairs per KV head, cdiv(ratio, 2): a workgroup serves one pair
-    int units;   // hkv * npairs: the grid's second dimension
-    int batch;        // rows of q / cached_lens (num_decoding[0] <= batch)
-    int head_fast;    // 1: grid (Hkv, pieces), the KV head in blockIdx.x; 0: grid (pieces, Hkv)
+    int ratio;    // query heads per KV head (GQA ratio, 1 ... 16)
+    int batch;    // rows of q / cached_lens (num_decoding[0] <= batch)
+    int out_vec;  // out rows take 8-byte stores
     // The fused form (ie_decode_attention_rope): q holds the QKV projection's raw rows, and the
     // launch does fused_rope_kv_decode's work itself: q normed, rotated and scaled by the
     // calibration as that kernel computes it, and the new token's K/V row quantized and written
@@ -194,175 +188,195 @@ struct DecodeArgs {
 };
 
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ v4u ld128(rsrc_t r, int off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, IE_DECODE_LOAD_AUX);
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int DA_TOK = 32;                      // tokens per block
+constexpr int DA_V = 4096, DA_SC = 8192;        // byte offsets in a stage: V rows, then scales
+constexpr int DA_STAGE = DA_SC + 2 * 4 * DA_TOK;
+constexpr int DA_QROW = DA_D + 8;               // LDS row of q (bf16), padded by 16 bytes
+constexpr int DA_OROW = DA_D + 4;               // LDS row of a wave's output (fp32), padded
+constexpr float DA_SLACK = 3.0f;  // the running max moves when a score exceeds it by 2^3
+// V scales served by the wave's exponent ve: [2^(5 - ve), 2^(12 - ve)); with p <= 2^(DA_SLACK + ve)
+// the fp16 products stay below 2^15
+constexpr int DA_VE_TOP = 12, DA_VE_WIN = 7;
+static_assert(16 * DA_OROW * 4 <= 2 * DA_STAGE, "a wave's output overlays its stages");
+
+// 16 (4) bytes per lane from memory to LDS at lds + 16 (4) lane, counted by vmcnt; lanes past the
+// descriptor's range touch no memory. In assembly so that the compiler's own waits do not drain
+// the stages in flight: the waits are the caller's. s_nop: m0 is read by the load.
+__device__ __forceinline__ void da_dma16(v4u rsrc, int off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                 :: "s"(lds), "v"(off), "s"(rsrc) : "memory", "m0");
+}
+__device__ __forceinline__ void da_dma4(const float* p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                 :: "s"(lds), "v"(p) : "memory", "m0");
+}
+constexpr int DA_DMAS = 9;  // per block: 4 K, 4 V, the scales
+__device__ __forceinline__ v4u da_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t p = (uint64_t)base;
+    return v4u{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, (uint32_t)RSRC_WORD3};
 }
 
-// Running softmax state of one lane: query heads (2hk, 2hk+1), channels [16c, 16c+16).
-// The PV products are fp16 values of p * v_scale * 2^ve: the exponent ve is chosen from the V
-// scales the lane group has seen so that the largest product stays inside fp16's normal range
-// whatever the magnitude of V (the reference rounds p * v_scale to bf16, whose exponent range
-// is fp32's). l, ps and acc all carry the factor 2^ve, so the state is an ordinary online
-// softmax whose running maximum m is kept as (max score - ve), and it merges as one.
-struct LaneState {
-    float m[2], l[2], ps[2];
-    float acc[2][16];
-    float ve;       // an integer
-    uint32_t vlo;   // bits of 2^(8 - ve): the V scales this ve serves are [2^(8-ve), 2^(15-ve))
-};
-
-// Registers of one 32-token block of a wave: lane group g holds tokens t0+4g .. t0+4g+3,
-// channels [16c, 16c+16), plus their 4 K (or V) scales.
-struct KVRegs {
-    v4u x[DA_U];
-    v4u scale;
-};
-
-__device__ __forceinline__ void load_block(KVRegs& r, rsrc_t rows, rsrc_t scales, int tok,
-                                           int cc) {
-    const int off = tok * DA_D + 16 * cc;
-#pragma unroll
-    for (int u = 0; u < DA_U; ++u) r.x[u] = ld128(rows, off + u * DA_D);
-    r.scale = ld128(scales, tok * 4);
+// eight int8 (two words) -> fp16, exactly
+__device__ __forceinline__ half8_t da_cvt8(uint32_t x0, uint32_t x1) {
+    const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    x0 ^= 0x80808080u;
+    x1 ^= 0x80808080u;
+    const half2_t a = as_h2(__builtin_amdgcn_perm(K64, x0, 0x04010400u)) - off;
+    const half2_t b = as_h2(__builtin_amdgcn_perm(K64, x0, 0x04030402u)) - off;
+    const half2_t c = as_h2(__builtin_amdgcn_perm(K64, x1, 0x04010400u)) - off;
+    const half2_t d = as_h2(__builtin_amdgcn_perm(K64, x1, 0x04030402u)) - off;
+    return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-// Scores of the block in base 2 up to the head's factor kmul (applied in block_pv):
-// t = (q.k - 1152 sum q) * k_scale, where q is q * 2^e in fp16 and kmul = scale * log2(e) / 2^e.
-// The 1152 sum q offset enters as the dot chain's starting value: qoff = -1152 sum q / 8 in
-// each of the 8 lanes of a row, which the row sum adds up. qoff and kmul are wave-uniform.
-// With MASKED, tokens at or past t_end score -inf (their loads returned zeros: buffer range).
+struct DecodeState {
+    f32x4_t acc[8];  // lane (r, g): head r, channel 32 g + 8 i + mm in acc[mm][i]
+    float m, l;      // head r: running max - ve (all four g lanes), sum of p over the lane's tokens
+    float ve;        // wave-uniform, an integer
+    uint32_t vlo;    // bits of 2^(5 - ve)
+};
+
+// One block in LDS stage `st`, first token t0; MASKED: tokens at or past t_end do not count.
 template <bool MASKED>
-__device__ __forceinline__ void block_scores(float (&t)[DA_U][2], const KVRegs& k,
-                                             const half2_t (&qh)[2][8], const float (&qoff)[2],
-                                             int tok, int t_end) {
+__device__ __forceinline__ void da_block(DecodeState& s, const half8_t (&qf)[4], float kmul,
+                                         const uint8_t* st, int t0, int t_end, int l16, int g) {
+    v4u k[2][2];
 #pragma unroll
-    for (int u = 0; u < DA_U; ++u) {
-        float d0 = qoff[0], d1 = qoff[1];
+    for (int mt = 0; mt < 2; ++mt) {
+        const uint8_t* row = st + (16 * mt + l16) * DA_D;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t x = k.x[u][i] ^ 0x80808080u;
-            const half2_t h01 = as_h2(__builtin_amdgcn_perm(K64, x, 0x04010400u));
-            const half2_t h23 = as_h2(__builtin_amdgcn_perm(K64, x, 0x04030402u));
-            d0 = fdot2(qh[0][2 * i], h01, d0);
-            d0 = fdot2(qh[0][2 * i + 1], h23, d0);
-            d1 = fdot2(qh[1][2 * i], h01, d1);
-            d1 = fdot2(qh[1][2 * i + 1], h23, d1);
-        }
-        d0 = sum8(d0);
-        d1 = sum8(d1);
-        const float ks = __uint_as_float(k.scale[u]);
-        t[u][0] = d0 * ks;
-        t[u][1] = d1 * ks;
-        if (MASKED && tok + u >= t_end) t[u][0] = t[u][1] = -INFINITY;
+        for (int c = 0; c < 2; ++c)
+            k[mt][c] = *reinterpret_cast<const v4u*>(row + (((g + 4 * c) ^ (l16 & 7)) << 4));
     }
-}
-
-// Online-softmax update of the lane group and the PV accumulation of the block; scores are
-// s = t * kmul (kmul > 0).
-__device__ __forceinline__ void block_pv(LaneState& st, const float (&t)[DA_U][2],
-                                         const KVRegs& v, const float (&kmul)[2]) {
-    // The block's largest V scale vmax lies in [2^(ex-1), 2^ex). With p <= 2^ve the products
-    // stay below 2^15 while vmax < 2^(15-ve); the exponent is re-chosen (ve = 15 - ex, so
-    // vmax * 2^ve lies in [2^14, 2^15)) when that fails, or when vmax < 2^(8-ve), i.e. the
-    // scales fell by 2^6 or more and small products would lose precision. Both bounds are one
-    // unsigned compare on the float bits. The state is rescaled by the exact power of two and
-    // m moves with ve. Scales past the piece's end load as 0 and change nothing.
-    const float vmax = fmaxf(fmaxf(__uint_as_float(v.scale[0]), __uint_as_float(v.scale[1])),
-                             fmaxf(__uint_as_float(v.scale[2]), __uint_as_float(v.scale[3])));
-    if (__float_as_uint(vmax) - st.vlo >= (7u << 23)) {
-        if (vmax > 0.0f) {
-            const int ex = __builtin_amdgcn_frexp_expf(vmax);
-            const float ve = (float)(15 - ex);
-            const float d = ve - st.ve;
-            const float r = ldexpf(1.0f, (int)d);
+    f32x4_t ks[2], vs[2];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+    for (int mt = 0; mt < 2; ++mt) {
+        ks[mt] = *reinterpret_cast<const f32x4_t*>(st + DA_SC + 4 * (16 * mt + 4 * g));
+        vs[mt] = *reinterpret_cast<const f32x4_t*>(st + DA_SC + 4 * (DA_TOK + 16 * mt + 4 * g));
+    }
+    uint2 v[8];  // the lane's 8 tokens, channels 8 r ... 8 r + 7
 #pragma unroll
-                for (int j = 0; j < 16; ++j) st.acc[h][j] *= r;
-                st.l[h] *= r;
-                st.ps[h] *= r;
-                st.m[h] -= d;  // -inf stays -inf
+    for (int u = 0; u < 8; ++u)
+        v[u] = *reinterpret_cast<const uint2*>(
+            st + DA_V + (16 * (u >> 2) + 4 * g + (u & 3)) * DA_D + 8 * l16);
+    f32x4_t x[2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+        f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                da_cvt8(k[mt][k4 >> 1][2 * (k4 & 1)], k[mt][k4 >> 1][2 * (k4 & 1) + 1]), qf[k4],
+                c, 0, 0, 0);
+        x[mt] = c * ks[mt];
+    }
+    if (MASKED) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool in = t0 + 16 * mt + 4 * g + i < t_end;
+                x[mt][i] = in ? x[mt][i] : -INFINITY;
+                vs[mt][i] = in ? vs[mt][i] : 0.0f;
             }
-            st.ve = ve;
-            st.vlo = (uint32_t)(ex - 7 + 127) << 23;
-        }
     }
-    float nms[2];  // minus the effective running max, the exp2 argument's offset
+    float mx = -INFINITY, vmax = 0.0f;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const float mt =
-            fmaxf(fmaxf(t[0][h], t[1][h]), fmaxf(t[2][h], t[3][h])) * kmul[h] - st.ve;
-        if (mt > st.m[h]) {
-            const float alpha = exp2_safe(st.m[h] - mt);  // m = -inf -> 0
-#pragma unroll
-            for (int j = 0; j < 16; ++j) st.acc[h][j] *= alpha;
-            st.l[h] *= alpha;
-            st.ps[h] *= alpha;
-            st.m[h] = mt;
-        }
-        // p = 2^(s - max + ve) <= 2^ve
-        nms[h] = st.m[h] == -INFINITY ? 0.0f : -st.m[h];
-    }
-    half2_t pp[DA_U / 2][2];  // (p * v_scale * 2^ve) of token pairs, fp16
-#pragma unroll
-    for (int pr = 0; pr < DA_U / 2; ++pr)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float pa = exp2_safe(__builtin_fmaf(t[2 * pr][h], kmul[h], nms[h]));
-            const float pb = exp2_safe(__builtin_fmaf(t[2 * pr + 1][h], kmul[h], nms[h]));
-            st.l[h] += pa + pb;
-            pp[pr][h] = half2_t{(_Float16)(pa * __uint_as_float(v.scale[2 * pr])),
-                                (_Float16)(pb * __uint_as_float(v.scale[2 * pr + 1]))};
-            st.ps[h] = fdot2(pp[pr][h], half2_t{(_Float16)1.0f, (_Float16)1.0f}, st.ps[h]);
-        }
-#pragma unroll
-    for (int pr = 0; pr < DA_U / 2; ++pr) {
-        const int ua = 2 * pr, ub = ua + 1;
+    for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t xa = v.x[ua][i] ^ 0x80808080u, xb = v.x[ub][i] ^ 0x80808080u;
+            mx = fmaxf(mx, x[mt][i]);
+            vmax = fmaxf(vmax, vs[mt][i]);
+        }
+    mx *= kmul;
+    // The rare, wave-uniform branch: the running max moves (a score more than DA_SLACK above it),
+    // or the V scales leave the window the exponent serves (one lane's above it, or all below).
+    if (__ballot(mx - s.ve > s.m + DA_SLACK ||
+                 __float_as_uint(vmax) >= s.vlo + ((uint32_t)DA_VE_WIN << 23)) ||
+        !__ballot(__float_as_uint(vmax) >= s.vlo)) {
+        const float vw = wave_max(vmax);
+        const uint32_t vb = __float_as_uint(vw);
+        if (vw > 0.0f && vb - s.vlo >= ((uint32_t)DA_VE_WIN << 23)) {
+            const int ex = __builtin_amdgcn_frexp_expf(vw);  // vw in [2^(ex-1), 2^ex)
+            const float ve = (float)(DA_VE_TOP - ex);
+            const float d = ve - s.ve, r = ldexpf(1.0f, (int)d);
+#pragma unroll
+            for (int mm = 0; mm < 8; ++mm) s.acc[mm] *= r;
+            s.l *= r;
+            s.m -= d;  // -inf stays -inf
+            s.ve = ve;
+            s.vlo = (uint32_t)(ex - DA_VE_WIN + 127) << 23;
+        }
+        const float rm = max_xor32(max_xor16(mx)) - s.ve;
+        if (rm > s.m + DA_SLACK) {
+            const float alpha = exp2_safe(s.m - rm);  // m = -inf -> 0
+#pragma unroll
+            for (int mm = 0; mm < 8; ++mm) s.acc[mm] *= alpha;
+            s.l *= alpha;
+            s.m = rm;
+        }
+    }
+    const float nms = s.m == -INFINITY ? 0.0f : -s.m;
+    half8_t p;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float e = exp2_safe(__builtin_fmaf(x[mt][i], kmul, nms));
+            s.l += e;
+            p[4 * mt + i] = (_Float16)(e * vs[mt][i]);
+        }
+    const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {  // channels 8 r + 4 w ... + 3
+        half2_t f[4][4];           // [channel][token pair]
+#pragma unroll
+        for (int u = 0; u < 8; u += 2) {
+            const uint32_t xa = (w ? v[u].y : v[u].x) ^ 0x80808080u;
+            const uint32_t xb = (w ? v[u + 1].y : v[u + 1].x) ^ 0x80808080u;
             const uint32_t t01 = __builtin_amdgcn_perm(xb, xa, 0x05010400u);
             const uint32_t t23 = __builtin_amdgcn_perm(xb, xa, 0x07030602u);
-            const half2_t c[4] = {as_h2(__builtin_amdgcn_perm(K64, t01, 0x04010400u)),
-                                  as_h2(__builtin_amdgcn_perm(K64, t01, 0x04030402u)),
-                                  as_h2(__builtin_amdgcn_perm(K64, t23, 0x04010400u)),
-                                  as_h2(__builtin_amdgcn_perm(K64, t23, 0x04030402u))};
+            f[0][u / 2] = as_h2(__builtin_amdgcn_perm(K64, t01, 0x04010400u)) - off;
+            f[1][u / 2] = as_h2(__builtin_amdgcn_perm(K64, t01, 0x04030402u)) - off;
+            f[2][u / 2] = as_h2(__builtin_amdgcn_perm(K64, t23, 0x04010400u)) - off;
+            f[3][u / 2] = as_h2(__builtin_amdgcn_perm(K64, t23, 0x04030402u)) - off;
+        }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                st.acc[0][4 * i + j] = fdot2(pp[pr][0], c[j], st.acc[0][4 * i + j]);
-                st.acc[1][4 * i + j] = fdot2(pp[pr][1], c[j], st.acc[1][4 * i + j]);
-            }
+        for (int c = 0; c < 4; ++c) {
+            const half8_t a = {f[c][0][0], f[c][0][1], f[c][1][0], f[c][1][1],
+                               f[c][2][0], f[c][2][1], f[c][3][0], f[c][3][1]};
+            s.acc[4 * w + c] =
+                __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p, s.acc[4 * w + c], 0, 0, 0);
         }
     }
 }
 
-#ifndef IE_DECODE_WAVES_PER_EU
-#define IE_DECODE_WAVES_PER_EU 4
-#endif
-
-// GQA2: the launch's GQA ratio is 2 (one query-head pair per KV head), so the pair's query
-// heads are 2 hk and 2 hk + 1 at compile time; other ratios take the generic form.
-template <int WAVES, bool ROPE, bool GQA2>
-__global__ __launch_bounds__(WAVES * IE_WAVE)
-__attribute__((amdgpu_waves_per_eu(IE_DECODE_WAVES_PER_EU))) void decode_attention_kernel(
-    DecodeArgs a) {
-    constexpr int THREADS = WAVES * IE_WAVE;
-    constexpr int TOK_WG = WAVES * DA_TOK_WAVE;  // tokens per workgroup step
-    const int lane0 = threadIdx.x & 63;
+// grid (nwork, Hkv), block 64 W.
+template <int W, bool ROPE>
+__global__ __launch_bounds__(W * IE_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+decode_attention_kernel(DecodeArgs a) {
+    constexpr int THREADS = W * IE_WAVE;
+    // q's rows of the fused form lie beside the stages; sixteen would cost a one-wave workgroup its
+    // eighth place on the CU, so it has eight, and more lie over the second stage, which is then
+    // requested after they are read
+    constexpr int Q_ROWS = !ROPE ? 1 : W == 1 ? 8 : 16;
+    const bool q_over = ROPE && W == 1 && a.ratio > Q_ROWS;
+    static_assert(16 * DA_QROW * 2 <= DA_STAGE, "q's rows fit a stage");
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring[W][2][DA_STAGE];
+    __shared__ __attribute__((aligned(16))) uint16_t s_qrow[Q_ROWS][DA_QROW];
+    __shared__ float s_m[W][16], s_l[W][16];
+    uint16_t(*s_q)[DA_QROW] =
+        q_over ? reinterpret_cast<uint16_t(*)[DA_QROW]>(s_ring[0][1]) : s_qrow;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
     // The first 64 sequences' lengths and cache slots, issued beside num_decoding: for them the
     // row to stream is known from registers once the work entry is found.
-    const int raw0 = lane0 < a.batch ? a.cached_lens[lane0] : 0;
-    const int slot0 = lane0 < a.batch ? a.slot_ids[lane0] : 0;
+    const int raw0 = lane < a.batch ? a.cached_lens[lane] : 0;
+    const int slot0 = lane < a.batch ? a.slot_ids[lane] : 0;
     const int nd = a.num_decoding[0];
-    // the workgroup's (KV head, query-head pair): query heads qh0 = ratio * hk + 2 * pair and
-    // qh0 + 1 (the pair of an odd ratio's last pair is one head: has2 = false)
-    const int hk = a.head_fast ? blockIdx.x : blockIdx.y;
-    const int pair = GQA2 ? 0 : (int)blockIdx.z;
-    const int item = a.head_fast ? blockIdx.y : blockIdx.x;
-    const int unit = GQA2 ? hk : hk * a.npairs + pair;
-    const int qh0 = GQA2 ? 2 * hk : uniform(a.ratio * hk + 2 * pair);
-    const bool has2 = GQA2 || 2 * pair + 1 < a.ratio;
-    const int qh1 = has2 ? qh0 + 1 : qh0;  // an absent second head repeats the first
+    const int item = blockIdx.x, hk = blockIdx.y, R = a.ratio, qh0 = R * hk;
     Work wk;
     if (a.plan) {  // one 16-byte row, requested with the loads above
         const int4 r = *reinterpret_cast<const int4*>(a.plan + 4 * item);
@@ -370,58 +384,56 @@ __attribute__((amdgpu_waves_per_eu(IE_DECODE_WAVES_PER_EU))) void decode_attenti
     } else {
         wk = decode_assign(a.cached_lens, nd, item, a.target, raw0);
     }
-    // Wave-uniform by construction; readfirstlane lets the compiler keep them (and the buffer
-    // descriptors built from them) in SGPRs.
-    wk.needed = uniform(wk.needed);
-    if (wk.needed == 0) return;
-    const int b = uniform(wk.b);
-    const int split = uniform(wk.split);
-    const int piece = uniform(wk.piece);
+    const int needed = uniform(wk.needed);
+    if (needed == 0) return;
+    const int b = uniform(wk.b), split = uniform(wk.split), piece = uniform(wk.piece);
     const int n_end =
         b < 64 ? __builtin_amdgcn_readlane(raw0, b) + 1 : uniform(a.cached_lens[b] + 1);
-    const int t_begin = split * piece;
     const int slot = b < 64 ? __builtin_amdgcn_readlane(slot0, b) : uniform(a.slot_ids[b]);
-    // In the fused form the piece that ends at the new token (the sequence's last) takes that
-    // token from registers, not from the cache it writes it to: it streams one token less.
-    const bool last = ROPE && split == wk.needed - 1;
-    const int t_end = min(t_begin + piece, n_end) - (last ? 1 : 0);
+    const int t_begin = split * piece, t_end = min(t_begin + piece, n_end);
 
-    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    const int g = lane >> 3, cc = lane & 7;
+    const v4u rk = da_rsrc(a.c.k + slot * a.c.stride_slot + hk * a.c.stride_head,
+                           (uint32_t)t_end * DA_D);
+    const v4u rv = da_rsrc(a.c.v + slot * a.c.stride_slot + hk * a.c.stride_head,
+                           (uint32_t)t_end * DA_D);
+    // lanes 0 ... 31: the block's K scales, lanes 32 ... 63 its V scales
+    const float* sc = (lane < DA_TOK ? a.c.k_scale : a.c.v_scale) +
+                      slot * a.c.scale_stride_slot + hk * a.c.scale_stride_head;
+    uint8_t* ring = s_ring[wave][0];
+    const uint32_t lds0 = (uint32_t)uniform(
+        (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring);
+    const int koff = (lane >> 3) * DA_D + (((lane & 7) ^ (lane >> 3)) << 4), voff = 16 * lane;
+    auto issue = [&](int stage, int t0) {
+        const uint32_t l = lds0 + stage * DA_STAGE;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) da_dma16(rk, t0 * DA_D + 1024 * i + koff, l + 1024 * i);
+        da_dma4(sc + min(t0 + (lane & (DA_TOK - 1)), t_end - 1), l + DA_SC);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            da_dma16(rv, t0 * DA_D + 1024 * i + voff, l + DA_V + 1024 * i);
+    };
+    // this wave's blocks: w, w + W, ... of the piece's 32-token blocks
+    const int nb = (t_end - t_begin + DA_TOK - 1) / DA_TOK;
+    const int cw = wave < nb ? (nb - wave + W - 1) / W : 0;
+    const int t_first = t_begin + wave * DA_TOK;
 
-    // Buffer resources over this (slot, kv head) row, bounded at the piece's end.
-    const int8_t* krow = a.c.k + slot * a.c.stride_slot + hk * a.c.stride_head;
-    const int8_t* vrow = a.c.v + slot * a.c.stride_slot + hk * a.c.stride_head;
-    const float* ksrow = a.c.k_scale + slot * a.c.scale_stride_slot + hk * a.c.scale_stride_head;
-    const float* vsrow = a.c.v_scale + slot * a.c.scale_stride_slot + hk * a.c.scale_stride_head;
-    const rsrc_t rk = make_rsrc(krow, (uint32_t)t_end * DA_D);
-    const rsrc_t rv = make_rsrc(vrow, (uint32_t)t_end * DA_D);
-    const rsrc_t rks = make_rsrc(ksrow, (uint32_t)t_end * 4);
-    const rsrc_t rvs = make_rsrc(vsrow, (uint32_t)t_end * 4);
-
-    // ---- q of the two heads of this KV head, channels [16cc, 16cc + 16) ----
-    half2_t qh[2][8];
-    float qoff[2], kmul[2];  // wave-uniform (kept in SGPRs)
-    uint4 qraw[2][2];
-    // Fused form, in fused_rope_kv_decode's layout (lane i holds channels i and i + 64): every
-    // wave norms and rotates both query heads itself and moves them to the decode layout
-    // through its own LDS rows (no workgroup barrier); the last wave of the last piece also
-    // quantizes the new K and V rows (rk1.. below) for the cache and for its own use.
-    uint16_t rq1[2], rq2[2], rqw1 = 0, rqw2 = 0, rcs = 0, rsn = 0;
+    // ---- q, and in the fused form the new token's K/V row ----
+    const bool last = ROPE && split == needed - 1;
+    const bool kv_wave = last && wave == (nb - 1) % W;  // the owner of the new token's block
+    uint4 qraw[4];  // lane (r, g): head r, channels 16 g ... + 15 and 64 + 16 g ... + 15
+    constexpr int RPW = 16 / W;  // query heads a wave norms and rotates, at most
+    uint16_t rq1[RPW], rq2[RPW], rqw1 = 0, rqw2 = 0, rcs = 0, rsn = 0;
     uint16_t rk1 = 0, rk2 = 0, rkw1 = 0, rkw2 = 0, rv1 = 0, rv2 = 0;
     float rc1 = 0.f, rc2 = 0.f;
-    // the new K/V row is written to the cache by the first pair's workgroup only (the others
-    // compute it for their own use)
-    const bool kv_wave = last && wave == WAVES - 1;
-    const bool kv_write = kv_wave && pair == 0;
     if constexpr (ROPE) {
         const float* cal =
             a.c.k_calibration + slot * a.c.cal_stride_slot + hk * a.c.cal_stride_head;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint16_t* src = a.q + b * a.q_sb + (h ? qh1 : qh0) * a.q_sh;
-            rq1[h] = src[lane];
-            rq2[h] = src[lane + 64];
+        for (int i = 0; i < RPW; ++i) {
+            const int h = min(wave + W * i, R - 1);
+            const uint16_t* src = a.q + b * a.q_sb + (qh0 + h) * a.q_sh;
+            rq1[i] = src[lane];
+            rq2[i] = src[lane + 64];
         }
         rqw1 = a.q_norm[lane];
         rqw2 = a.q_norm[lane + 64];
@@ -440,38 +452,33 @@ __attribute__((amdgpu_waves_per_eu(IE_DECODE_WAVES_PER_EU))) void decode_attenti
             rv2 = vp[lane + 64];
         }
     } else {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint16_t* qp = a.q + b * a.q_sb + (h ? qh1 : qh0) * a.q_sh + 16 * cc;
-            qraw[h][0] = *reinterpret_cast<const uint4*>(qp);
-            qraw[h][1] = *reinterpret_cast<const uint4*>(qp + 8);
-        }
+        const uint16_t* qp = a.q + b * a.q_sb + (qh0 + min(l16, R - 1)) * a.q_sh + 16 * g;
+        qraw[0] = *reinterpret_cast<const uint4*>(qp);
+        qraw[1] = *reinterpret_cast<const uint4*>(qp + 8);
+        qraw[2] = *reinterpret_cast<const uint4*>(qp + 64);
+        qraw[3] = *reinterpret_cast<const uint4*>(qp + 72);
     }
-    // The first K/V block is requested with q, in the same memory round trip; the scheduling
-    // barrier keeps the compiler from sinking the requests below q's conversion.
-    int t0 = t_begin + wave * DA_TOK_WAVE;
-    KVRegs kr, vr;
-    load_block(kr, rk, rks, t0 + 4 * g, cc);
-    load_block(vr, rv, rvs, t0 + 4 * g, cc);
     __builtin_amdgcn_sched_barrier(0);
-    __shared__ __attribute__((aligned(16))) uint16_t s_q[ROPE ? WAVES : 1][2][DA_D];
-    __shared__ __attribute__((aligned(16))) int8_t s_new[2][DA_D];
-    __shared__ float s_new_scale[2];
+    if (cw > 0) issue(0, t_first);
+    // q and the first block share a round trip; the second block is requested once q is here
+    // (the compiler's wait for q drains what was requested before it)
+    int32_t nk1 = 0, nk2 = 0, nv1 = 0, nv2 = 0;
+    float nks = 0.f, nvs = 0.f;
     if constexpr (ROPE) {
-        // fused_rope_kv_decode's arithmetic (the same device functions): RMSNorm and RoPE, q
-        // times the calibration rounded to bf16, K divided by the calibration, K and V
-        // quantized; the new row goes to the cache at column n_end - 1 and, with its scales,
-        // to LDS for the last wave's own use
+        asm volatile("" :: "v"(rq1[0]), "v"(rc2) : "memory");
+        if (!q_over && cw > 1) issue(1, t_first + W * DA_TOK);
         const float cs = bf16_to_f32(rcs), sn = bf16_to_f32(rsn);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int i = 0; i < RPW; ++i) {
+            const int h = wave + W * i;
+            if (h >= R) break;
             float o1, o2;
-            norm_rope_row(bf16_to_f32(rq1[h]), bf16_to_f32(rq2[h]), bf16_to_f32(rqw1),
+            norm_rope_row(bf16_to_f32(rq1[i]), bf16_to_f32(rq2[i]), bf16_to_f32(rqw1),
                           bf16_to_f32(rqw2), cs, sn, a.eps, o1, o2);
-            s_q[wave][h][lane] = (uint16_t)f32_to_bf16_rne(o1 * rc1);
-            s_q[wave][h][lane + 64] = (uint16_t)f32_to_bf16_rne(o2 * rc2);
+            s_q[h][lane] = (uint16_t)f32_to_bf16_rne(o1 * rc1);
+            s_q[h][lane + 64] = (uint16_t)f32_to_bf16_rne(o2 * rc2);
         }
-        if (kv_wave) {
+        if (kv_wave) {  // fused_rope_kv_decode's arithmetic; column n_end - 1 of the cache
             const int64_t col = n_end - 1;
             const int64_t base =
                 slot * a.c.stride_slot + hk * a.c.stride_head + col * a.c.stride_tok;
@@ -479,277 +486,193 @@ __attribute__((amdgpu_waves_per_eu(IE_DECODE_WAVES_PER_EU))) void decode_attenti
             float o1, o2;
             norm_rope_row(bf16_to_f32(rk1), bf16_to_f32(rk2), bf16_to_f32(rkw1),
                           bf16_to_f32(rkw2), cs, sn, a.eps, o1, o2);
-            int32_t q1, q2;
-            const float sk = quantize_row_wave(o1 / rc1, o2 / rc2, q1, q2);
-            if (kv_write) {
-                a.c.k[base + lane] = (int8_t)q1;
-                a.c.k[base + lane + 64] = (int8_t)q2;
-            }
-            s_new[0][lane] = (int8_t)q1;
-            s_new[0][lane + 64] = (int8_t)q2;
-            const float sv = quantize_row_wave(bf16_to_f32(rv1), bf16_to_f32(rv2), q1, q2);
-            if (kv_write) {
-                a.c.v[base + lane] = (int8_t)q1;
-                a.c.v[base + lane + 64] = (int8_t)q2;
-            }
-            s_new[1][lane] = (int8_t)q1;
-            s_new[1][lane + 64] = (int8_t)q2;
+            nks = quantize_row_wave(o1 / rc1, o2 / rc2, nk1, nk2);
+            nvs = quantize_row_wave(bf16_to_f32(rv1), bf16_to_f32(rv2), nv1, nv2);
+            a.c.k[base + lane] = (int8_t)nk1;
+            a.c.k[base + lane + 64] = (int8_t)nk2;
+            a.c.v[base + lane] = (int8_t)nv1;
+            a.c.v[base + lane + 64] = (int8_t)nv2;
             if (lane == 0) {
-                if (kv_write) {
-                    a.c.k_scale[sidx] = sk;
-                    a.c.v_scale[sidx] = sv;
-                }
-                s_new_scale[0] = sk;
-                s_new_scale[1] = sv;
+                a.c.k_scale[sidx] = nks;
+                a.c.v_scale[sidx] = nvs;
             }
         }
-        // the wave's own LDS rows: its writes are visible to its later reads once the LDS
-        // operations are ordered within the wave
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            qraw[h][0] = *reinterpret_cast<const uint4*>(&s_q[wave][h][16 * cc]);
-            qraw[h][1] = *reinterpret_cast<const uint4*>(&s_q[wave][h][16 * cc + 8]);
+        __syncthreads();
+        const uint16_t* qp = &s_q[min(l16, R - 1)][16 * g];
+        qraw[0] = *reinterpret_cast<const uint4*>(qp);
+        qraw[1] = *reinterpret_cast<const uint4*>(qp + 8);
+        qraw[2] = *reinterpret_cast<const uint4*>(qp + 64);
+        qraw[3] = *reinterpret_cast<const uint4*>(qp + 72);
+        if (q_over && cw > 1) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(1, t_first + W * DA_TOK);
         }
+    } else {
+        asm volatile("" :: "v"(qraw[0].x), "v"(qraw[3].w) : "memory");
+        if (cw > 1) issue(1, t_first + W * DA_TOK);
     }
+    half8_t qf[4];
+    float kmul;
+    {
+        float f[4][8], amax = 0.0f;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const uint4 u0 = qraw[h][0], u1 = qraw[h][1];
-        const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-        float f[16];
-        float amax = 0.0f;
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t w[4] = {qraw[i].x, qraw[i].y, qraw[i].z, qraw[i].w};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            f[2 * i] = bf16lo(w[i]);
-            f[2 * i + 1] = bf16hi(w[i]);
-            amax = fmaxf(amax, fmaxf(fabsf(f[2 * i]), fabsf(f[2 * i + 1])));
+            for (int j = 0; j < 4; ++j) {
+                f[i][2 * j] = bf16lo(w[j]);
+                f[i][2 * j + 1] = bf16hi(w[j]);
+                amax = fmaxf(amax, fmaxf(fabsf(f[i][2 * j]), fabsf(f[i][2 * j + 1])));
+            }
         }
-        amax = fmaxf(amax, dpp<DPP_XOR1>(amax));
-        amax = fmaxf(amax, dpp<DPP_XOR2>(amax));
-        amax = fmaxf(amax, dpp<DPP_HALF_MIRROR>(amax));
+        amax = max_xor32(max_xor16(amax));
         int e = 0;
         frexpf(amax, &e);
-        const float sc = amax > 0.0f ? ldexpf(1.0f, 14 - e) : 1.0f;  // amax*sc in [2^13, 2^14)
-        float s = 0.0f;
+        const float scl = amax > 0.0f ? ldexpf(1.0f, 14 - e) : 1.0f;  // amax scl in [2^13, 2^14)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const _Float16 lo = (_Float16)(f[2 * i] * sc), hi = (_Float16)(f[2 * i + 1] * sc);
-            qh[h][i] = half2_t{lo, hi};
-            s += (float)lo + (float)hi;
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) qf[i][j] = (_Float16)(f[i][j] * scl);
+        kmul = a.scale_log2 / scl;
+    }
+
+    DecodeState s;
+#pragma unroll
+    for (int mm = 0; mm < 8; ++mm) s.acc[mm] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    s.m = -INFINITY;
+    s.l = 0.0f;
+    s.ve = 0.0f;
+    s.vlo = (uint32_t)(DA_VE_TOP - DA_VE_WIN + 127) << 23;
+    for (int j = 0, t0 = t_first; j < cw; ++j, t0 += W * DA_TOK) {
+        // block j is here once at most block j + 1's loads (if any) are outstanding
+        if (j + 1 < cw) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(DA_DMAS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint8_t* st = ring + (j & 1) * DA_STAGE;
+        if (t0 + DA_TOK <= t_end && !(kv_wave && j == cw - 1)) {
+            da_block<false>(s, qf, kmul, st, t0, t_end, l16, g);
+        } else {
+            if (kv_wave) {  // the new token's row takes the place of the cache column's old bytes
+                const int t = n_end - 1 - t0;
+                uint8_t* kr = st + t * DA_D;
+                kr[((((lane >> 4)) ^ (t & 7)) << 4) + l16] = (uint8_t)nk1;
+                kr[((((lane >> 4) + 4) ^ (t & 7)) << 4) + l16] = (uint8_t)nk2;
+                st[DA_V + t * DA_D + lane] = (uint8_t)nv1;
+                st[DA_V + t * DA_D + lane + 64] = (uint8_t)nv2;
+                if (lane == 0) {
+                    reinterpret_cast<float*>(st + DA_SC)[t] = nks;
+                    reinterpret_cast<float*>(st + DA_SC)[DA_TOK + t] = nvs;
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+            da_block<true>(s, qf, kmul, st, t0, t_end, l16, g);
         }
-        qoff[h] = __int_as_float(uniform(__float_as_int(sum8(s) * (-OFFSET / 8.0f))));
-        kmul[h] = __int_as_float(uniform(__float_as_int(a.scale_log2 / sc)));
-    }
-
-    LaneState st;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        st.m[h] = -INFINITY;
-        st.l[h] = 0.0f;
-        st.ps[h] = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) st.acc[h][j] = 0.0f;
-    }
-    st.ve = 0.0f;
-    st.vlo = (uint32_t)(8 + 127) << 23;
-
-    // Rolling pipeline: the next block's K is requested as soon as this block's scores are
-    // done and its V as soon as this block's PV is done, so every load has half a block of
-    // VALU work to hide behind without extra registers. Requests past the piece's end fall
-    // outside the buffer range and return zeros without touching memory.
-    // this wave's blocks: w, w + 8, ... of the piece's 32-token blocks, counted up front
-    const int nb = (t_end - t_begin + DA_TOK_WAVE - 1) / DA_TOK_WAVE;
-    const int cw = wave < nb ? (nb - wave + WAVES - 1) / WAVES : 0;
-    int nfull = cw;
-    if (cw > 0 && t_begin + DA_TOK_WAVE * (wave + WAVES * (cw - 1)) + DA_TOK_WAVE > t_end)
-        --nfull;  // the piece's last, partial block
-    float s[DA_U][2];
-    for (int j = 0; j < nfull; ++j, t0 += TOK_WG) {
-        block_scores<false>(s, kr, qh, qoff, t0 + 4 * g, t_end);
-        load_block(kr, rk, rks, t0 + TOK_WG + 4 * g, cc);
-        block_pv(st, s, vr, kmul);
-        load_block(vr, rv, rvs, t0 + TOK_WG + 4 * g, cc);
-    }
-    // the lane group derived afresh from the thread index for the masked blocks below: kept
-    // from the prologue it is a register the loop needs
-    int tid_m = lane_id();
-    asm volatile("" : "+v"(tid_m));
-    tid_m += IE_WAVE * wave;
-    const int gm = (tid_m & 63) >> 3;
-    if (nfull < cw) {
-        block_scores<true>(s, kr, qh, qoff, t0 + 4 * gm, t_end);
-        block_pv(st, s, vr, kmul);
-    }
-    if (ROPE && kv_wave) {
-        // the new token, as a block whose other tokens are masked: lane group 0 holds its row
-        KVRegs kn, vn;
-#pragma unroll
-        for (int u = 0; u < DA_U; ++u) kn.x[u] = vn.x[u] = v4u{0u, 0u, 0u, 0u};
-        kn.scale = vn.scale = v4u{0u, 0u, 0u, 0u};
-        if (gm == 0) {
-            const int cm = tid_m & 7;
-            kn.x[0] = *reinterpret_cast<const v4u*>(&s_new[0][16 * cm]);
-            vn.x[0] = *reinterpret_cast<const v4u*>(&s_new[1][16 * cm]);
-            kn.scale[0] = __float_as_uint(s_new_scale[0]);
-            vn.scale[0] = __float_as_uint(s_new_scale[1]);
-        }
-        block_scores<true>(s, kn, qh, qoff, n_end - 1 + 4 * gm, n_end);
-        block_pv(st, s, vn, kmul);
-    }
-
-    float (&m)[2] = st.m;
-    float (&l)[2] = st.l;
-    float (&ps)[2] = st.ps;
-    float (&acc)[2][16] = st.acc;
-
-    // ---- merge the 8 lane groups of the wave ----
-    float mw[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        float mx = m[h];
-        mx = fmaxf(mx, dpp<DPP_ROR8>(mx));
-        mx = fmaxf(mx, shfl_xor(mx, 16));
-        mx = fmaxf(mx, shfl_xor(mx, 32));
-        mw[h] = mx;
-        const float f = m[h] == -INFINITY ? 0.0f : exp2_safe(m[h] - mx);
-        float lf = l[h] * f;
-        lf += dpp<DPP_ROR8>(lf);
-        lf += shfl_xor(lf, 16);
-        lf += shfl_xor(lf, 32);
-        l[h] = lf;
-        const float off = ps[h] * OFFSET;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            float x = (acc[h][j] - off) * f;
-            x += dpp<DPP_ROR8>(x);
-            x += shfl_xor(x, 16);
-            x += shfl_xor(x, 32);
-            acc[h][j] = x;
+        if (j + 2 < cw) {  // every read of this stage has its data
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(j & 1, t0 + 2 * W * DA_TOK);
         }
     }
 
-    // ---- merge the waves through LDS ----
-    __shared__ float s_acc[WAVES][2][DA_D];
-    __shared__ float s_m[WAVES][2], s_l[WAVES][2];
-    // the lane's channel group, derived afresh from the thread index: keeping the prologue's copy
-    // alive across the loop costs a register the loop needs
-    int tid = lane_id();
-    asm volatile("" : "+v"(tid));
-    tid += IE_WAVE * wave;
-    const int ccm = tid & 7;
+    // ---- merge the waves through LDS (each wave's output over its own, drained stages) ----
+    s.l = sum_xor32(sum_xor16(s.l));
+    float* so = reinterpret_cast<float*>(ring);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            *reinterpret_cast<f32x4_t*>(so + l16 * DA_OROW + 32 * g + 8 * i + 4 * q) =
+                f32x4_t{s.acc[4 * q][i], s.acc[4 * q + 1][i], s.acc[4 * q + 2][i],
+                        s.acc[4 * q + 3][i]};
     if (g == 0) {
+        s_m[wave][l16] = s.m;
+        s_l[wave][l16] = s.l;
+    }
+    __syncthreads();
+    auto store_out = [&](int h, int d, f32x4_t y) {
+        uint16_t* o = a.out + b * a.o_sb + (qh0 + h) * a.o_sh + d;
+        if (a.out_vec) {
+            *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+        } else {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+            for (int i = 0; i < 4; ++i) o[i] = (uint16_t)f32_to_bf16_rne(y[i]);
+        }
+    };
+    // four channels of one head per thread and pass
+    const int quads = R * (DA_D / 4);
+    for (int q = tid; q < quads; q += THREADS) {
+        const int h = q >> 5, d = 4 * (q & 31);
+        float mx = -INFINITY;
 #pragma unroll
-            for (int j = 0; j < 16; ++j) s_acc[wave][h][16 * ccm + j] = acc[h][j];
-            if (ccm == 0) {
-                s_m[wave][h] = mw[h];
-                s_l[wave][h] = l[h];
+        for (int w = 0; w < W; ++w) mx = fmaxf(mx, s_m[w][h]);
+        f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float mw = s_m[w][h];
+            const float f = mw == -INFINITY ? 0.0f : exp2_safe(mw - mx);
+            num += *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(s_ring[w][0]) +
+                                                     h * DA_OROW + d) * f;
+            den += s_l[w][h] * f;
+        }
+        if (needed == 1) {
+            store_out(h, d, num / den);
+        } else {
+            const int64_t row = (int64_t)(qh0 + h) * a.nwork + item;
+            float* pa = a.part_acc + row * DA_D + d;
+            st_dev64(pa, (uint64_t)__float_as_uint(num[0]) | ((uint64_t)__float_as_uint(num[1]) << 32));
+            st_dev64(pa + 2, (uint64_t)__float_as_uint(num[2]) | ((uint64_t)__float_as_uint(num[3]) << 32));
+            if (d == 0) {
+                st_dev(a.part_m + row, mx);
+                st_dev(a.part_l + row, den);
             }
         }
     }
-    __syncthreads();
-    // one (query head, channel) output per thread, or two with 2-wave workgroups; threads past
-    // the 256 outputs stay for the barriers
-    constexpr int PER = (2 * DA_D + THREADS - 1) / THREADS;
-    float num[PER], den[PER], mxo[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-        const int idx = tid + u * THREADS;
-        const int h = (idx >> 7) & 1, d = idx & 127;
-        float mx = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, s_m[w][h]);
-        num[u] = 0.0f;
-        den[u] = 0.0f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float mwv = s_m[w][h];
-            const float f = mwv == -INFINITY ? 0.0f : exp2_safe(mwv - mx);
-            num[u] += s_acc[w][h][d] * f;
-            den[u] += s_l[w][h] * f;
-        }
-        mxo[u] = mx;
-    }
-    auto out_of = [&](int u) {
-        const int idx = tid + u * THREADS;
-        return a.out + b * a.o_sb + (qh0 + ((idx >> 7) & 1)) * a.o_sh + (idx & 127);
-    };
-    // thread idx's output exists (the second head of a one-head pair does not)
-    auto active = [&](int u) {
-        const int idx = tid + u * THREADS;
-        return idx < (has2 ? 2 : 1) * DA_D;
-    };
-    if (wk.needed == 1) {
-#pragma unroll
-        for (int u = 0; u < PER; ++u)
-            if (active(u)) *out_of(u) = (uint16_t)f32_to_bf16_rne(num[u] / den[u]);
-        return;
-    }
-    // A sequence of several pieces: each piece publishes its partial (the sequence's pieces
-    // are consecutive work entries) and counts itself in; the piece that arrives last merges
-    // them all (kernels.py:216-264, in base 2, pieces in order) and resets the count for the
-    // next call. The partials are written and read with device-coherent accesses.
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-        if (!active(u)) continue;
-        const int idx = tid + u * THREADS;
-        const int d = idx & 127;
-        const int64_t row = (int64_t)(qh0 + ((idx >> 7) & 1)) * a.nwork + item;
-        st_dev(a.part_acc + row * DA_D + d, num[u]);
-        if (d == 0) {
-            st_dev(a.part_m + row, mxo[u]);
-            st_dev(a.part_l + row, den[u]);
-        }
-    }
-    if (!arrive_last(a.arrivals + b * a.units + unit, wk.needed)) return;
-    const int needed = wk.needed;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-        if (!active(u)) continue;
-        const int idx = tid + u * THREADS;
-        const int d = idx & 127;
-        const int64_t row0 = (int64_t)(qh0 + ((idx >> 7) & 1)) * a.nwork + (item - split);
-        constexpr int CB = 8;  // partials per load batch: one memory round trip each
-        float av[CB], ml[CB][2];
+    if (needed == 1) return;
+    // A sequence of several pieces (consecutive work entries): each has published its partial with
+    // device-coherent stores and counts itself in; the last to arrive merges them all
+    // (kernels.py:216-264, in base 2, pieces in order) and resets the count for the next call.
+    if (!arrive_last(a.arrivals + b * a.hkv + hk, needed)) return;
+    const rsrc_t pr = make_rsrc(a.part_acc, (uint32_t)((int64_t)a.hq * a.nwork * DA_D * 4));
+    for (int q = tid; q < quads; q += THREADS) {
+        const int h = q >> 5, d = 4 * (q & 31);
+        const int64_t row0 = (int64_t)(qh0 + h) * a.nwork + (item - split);
+        constexpr int CB = 8;  // partials in flight: one round trip each batch
+        f32x4_t av[CB];
+        float pm[CB], pl[CB];
         auto load_batch = [&](int s0) {
 #pragma unroll
             for (int v = 0; v < CB; ++v) {
                 const bool in = s0 + v < needed;
-                av[v] = in ? ld_dev(a.part_acc + (row0 + s0 + v) * DA_D + d) : 0.0f;
-                ml[v][0] = in ? ld_dev(a.part_m + row0 + s0 + v) : -INFINITY;
-                ml[v][1] = in ? ld_dev(a.part_l + row0 + s0 + v) : 0.0f;
+                av[v] = __builtin_bit_cast(
+                    f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                 pr, in ? (int)(((row0 + s0 + v) * DA_D + d) * 4) : -64, 0, CPOL_SC1));
+                pm[v] = in ? ld_dev(a.part_m + row0 + s0 + v) : -INFINITY;
+                pl[v] = in ? ld_dev(a.part_l + row0 + s0 + v) : 0.0f;
             }
         };
-        // the largest partial maximum; with at most CB pieces the batch loaded here is the
-        // only one the merge needs
         load_batch(0);
-        float pm = -INFINITY;
+        float mx = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < CB; ++v) pm = fmaxf(pm, ml[v][0]);
+        for (int v = 0; v < CB; ++v) mx = fmaxf(mx, pm[v]);
         for (int s0 = CB; s0 < needed; s0 += CB) {
             float mv[CB];
 #pragma unroll
             for (int v = 0; v < CB; ++v)
                 mv[v] = s0 + v < needed ? ld_dev(a.part_m + row0 + s0 + v) : -INFINITY;
 #pragma unroll
-            for (int v = 0; v < CB; ++v) pm = fmaxf(pm, mv[v]);
+            for (int v = 0; v < CB; ++v) mx = fmaxf(mx, mv[v]);
         }
-        float nm = 0.0f, dn = 0.0f;
+        f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.0f;
         for (int s0 = 0; s0 < needed; s0 += CB) {
             if (s0 > 0) load_batch(s0);
 #pragma unroll
             for (int v = 0; v < CB; ++v) {
-                if (s0 + v < needed) {
-                    const float f = ml[v][0] == -INFINITY ? 0.0f : exp2_safe(ml[v][0] - pm);
-                    nm += av[v] * f;
-                    dn += ml[v][1] * f;
-                }
+                const float f = pm[v] == -INFINITY ? 0.0f : exp2_safe(pm[v] - mx);
+                num += av[v] * f;
+                den += pl[v] * f;
             }
         }
-        *out_of(u) = (uint16_t)f32_to_bf16_rne(nm / dn);
+        store_out(h, d, num / den);
     }
 }
 
@@ -833,17 +756,15 @@ struct Layout {
     size_t arr_off, acc_off, m_off, l_off, bytes;
 };
 
-// The layout of a launch of `units` units (decode_units). The count region has a count per
-// sequence and query head, the most any GQA ratio needs (one per sequence and unit), so every
-// launch of a batch size finds its counts and partials at the same offsets; the partial rows
-// (one per query head and work entry) fit the largest grid any ratio launches, that of
-// cdiv(hq, 2) units (workspace_size_layout).
-static Layout workspace_layout(int batch, int hq, int units) {
+// The layout of a launch whose entries are cut for `units` units. The count region has a count per
+// sequence and query head (a launch uses one per sequence and KV head), so every launch of a batch
+// size finds its counts and partials at the same offsets; then the partial rows, one per query
+// head and work entry.
+static Layout layout_of(int batch, int hq, int waves, int target) {
     Layout L;
-    batch = std::max(batch, 0);
-    L.waves = decode_waves(batch, units);
-    L.target = decode_target(units, L.waves);
-    L.nwork = batch <= L.target ? L.target : L.target + batch;
+    L.waves = waves;
+    L.target = target;
+    L.nwork = batch <= target ? target : target + batch;
     const size_t rows = (size_t)hq * L.nwork;
     L.arr_off = 0;
     L.acc_off = ((size_t)std::max(batch, DA_COUNT_CAP) * std::max(hq, DA_COUNT_HEADS) *
@@ -853,8 +774,35 @@ static Layout workspace_layout(int batch, int hq, int units) {
     L.bytes = L.l_off + rows * sizeof(float);
     return L;
 }
+static Layout workspace_layout(int batch, int hq, int units) {
+    batch = std::max(batch, 0);
+    const int waves = decode_waves(batch, units);
+    return layout_of(batch, hq, waves, decode_target(units, waves));
+}
+// What ie_decode_attention_workspace_size reserves: the larger of the grids of cdiv(hq, 2) units
+// (ratio 2) and of min(8, cdiv(hq, 2)) units, which gives launches above ratio 2 their entries.
 static Layout workspace_size_layout(int batch, int hq) {
-    return workspace_layout(batch, hq, std::max(1, (hq + 1) / 2));
+    const int pairs = std::max(1, (hq + 1) / 2);
+    const Layout a = workspace_layout(batch, hq, pairs);
+    const Layout b = workspace_layout(batch, hq, std::min(8, pairs));
+    return b.bytes > a.bytes ? b : a;
+}
+
+// The layout of a call. Ratios 1 and 2: the grid of their work lists (decode_units is Hkv). Above:
+// the same rule per KV head, but the partials of all heads of an entry must fit the workspace of
+// workspace_size_layout (and max_bytes, what the call may count on at most): where they do not,
+// workgroups of twice the waves and half the entries, up to 8 waves (one per CU), then as many
+// entries as fit (few KV heads only: at 8 the first rule always fits).
+static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes) {
+    if (hq <= 2 * hkv) return workspace_layout(batch, hq, hkv);
+    const Layout S = workspace_size_layout(batch, hq);
+    const size_t room = std::min(S.bytes, max_bytes), row = (DA_D + 2) * sizeof(float);
+    const int fit = room > S.acc_off ? (int)((room - S.acc_off) / (hq * row)) : 0;
+    auto entries = [&](int t) { return batch <= t ? t : t + batch; };
+    int waves = decode_waves(batch, hkv), target = decode_target(hkv, waves);
+    while (entries(target) > fit && waves < 8) target = decode_target(hkv, waves *= 2);
+    if (entries(target) > fit) target = std::max(1, batch <= fit ? fit : fit - batch);
+    return layout_of(batch, hq, waves, target);
 }
 
 }  // namespace ie
@@ -868,7 +816,7 @@ extern "C" size_t ie_decode_attention_workspace_counts_bytes(int32_t batch,
 }
 
 extern "C" int32_t ie_decode_attention_max_splits(int32_t num_units) {
-    return decode_target(num_units, 2);  // the largest target of any launch shape
+    return decode_target(num_units, 1);  // the largest target of any launch shape
 }
 
 extern "C" int32_t ie_decode_attention_target(int32_t batch, int32_t num_units) {
@@ -889,7 +837,8 @@ static hipError_t check_decode(const ie_bf16* q, int32_t batch, int32_t num_q_he
                                const ie_kv_cache* cache, const int32_t* cached_lens,
                                const int32_t* slot_ids, const int32_t* num_decoding,
                                const ie_bf16* out, int64_t q_sb, int64_t q_sh, void* workspace,
-                               size_t workspace_bytes, Layout* L, bool q_rows16 = true) {
+                               size_t workspace_bytes, Layout* L, bool q_rows16 = true,
+                               size_t max_bytes = SIZE_MAX) {
     hipError_t e = check_cache(cache);
     if (e != hipSuccess) return e;
     IE_REQUIRE(batch >= 0, "negative batch");
@@ -901,8 +850,7 @@ static hipError_t check_decode(const ie_bf16* q, int32_t batch, int32_t num_q_he
     IE_REQUIRE(!q_rows16 ||
                    ((reinterpret_cast<uintptr_t>(q) & 15) == 0 && q_sb % 8 == 0 && q_sh % 8 == 0),
                "q rows must be 16-byte aligned with contiguous head_dim");
-    *L = workspace_layout(batch, num_q_heads,
-                          decode_units(num_q_heads, (int)cache->num_kv_heads));
+    *L = call_layout(batch, num_q_heads, (int)cache->num_kv_heads, max_bytes);
     IE_REQUIRE(workspace != nullptr && workspace_bytes >= L->bytes, "workspace too small");
     IE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "workspace must be aligned");
     return hipSuccess;
@@ -937,48 +885,32 @@ static DecodeArgs decode_args(const ie_bf16* q, int64_t q_stride_b, int64_t q_st
     a.hq = num_q_heads;
     a.hkv = (int)cache->num_kv_heads;
     a.ratio = num_q_heads / a.hkv;
-    a.npairs = (a.ratio + 1) / 2;
-    a.units = a.hkv * a.npairs;
     a.batch = batch;
     return a;
 }
 
 template <bool ROPE>
-static hipError_t decode_launch(DecodeArgs& a, const Layout& L, int32_t batch,
-                                const ie_kv_cache* cache, hipStream_t stream) {
+static hipError_t decode_launch(DecodeArgs& a, const Layout& L, hipStream_t stream) {
     // pieces number at most target + nd, and at most target when nd <= target (decode_piece):
     // with batch <= target the grid needs no spare workgroups, which would otherwise hold
     // resident slots while they find out that they are idle
-    const unsigned pieces = (unsigned)L.nwork;
-    // The order in which the dispatcher hands out workgroups (same results either way): the KV
-    // heads of one piece side by side measured 9 % faster at B=64 ctx=1024, but 0.4-0.8 %
-    // slower at B=64 ctx=4096 and 3-4 % slower at config 5 (B=32); the host cannot tell the
-    // context lengths apart, so the pieces of one head go side by side unless
-    // IE_DECODE_HEAD_FAST_MIN_BATCH (0: never) is set.
-    a.head_fast = IE_DECODE_HEAD_FAST_MIN_BATCH > 0 && batch >= IE_DECODE_HEAD_FAST_MIN_BATCH &&
-                  pieces <= 65535;  // the grid's y dimension holds at most 65535
-    const dim3 grid = a.head_fast ? dim3((unsigned)a.hkv, pieces, (unsigned)a.npairs)
-                                  : dim3(pieces, (unsigned)a.hkv, (unsigned)a.npairs);
-    if (a.ratio == 2) {
-        switch (L.waves) {
-            case 8: hipLaunchKernelGGL((decode_attention_kernel<8, ROPE, true>), grid, dim3(512), 0, stream, a); break;
-            case 4: hipLaunchKernelGGL((decode_attention_kernel<4, ROPE, true>), grid, dim3(256), 0, stream, a); break;
-            default: hipLaunchKernelGGL((decode_attention_kernel<2, ROPE, true>), grid, dim3(128), 0, stream, a); break;
-        }
-    } else {
-        switch (L.waves) {
-            case 8: hipLaunchKernelGGL((decode_attention_kernel<8, ROPE, false>), grid, dim3(512), 0, stream, a); break;
-            case 4: hipLaunchKernelGGL((decode_attention_kernel<4, ROPE, false>), grid, dim3(256), 0, stream, a); break;
-            default: hipLaunchKernelGGL((decode_attention_kernel<2, ROPE, false>), grid, dim3(128), 0, stream, a); break;
-        }
+    const dim3 grid((unsigned)L.nwork, (unsigned)a.hkv);
+    a.out_vec = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && a.o_sb % 4 == 0 && a.o_sh % 4 == 0;
+    if (a.ratio > 2) a.plan = nullptr;  // a list of other entries (decode_units)
+    switch (L.waves) {
+        case 8: hipLaunchKernelGGL((decode_attention_kernel<8, ROPE>), grid, dim3(512), 0, stream, a); break;
+        case 4: hipLaunchKernelGGL((decode_attention_kernel<4, ROPE>), grid, dim3(256), 0, stream, a); break;
+        case 2: hipLaunchKernelGGL((decode_attention_kernel<2, ROPE>), grid, dim3(128), 0, stream, a); break;
+        default: hipLaunchKernelGGL((decode_attention_kernel<1, ROPE>), grid, dim3(64), 0, stream, a); break;
     }
     return hipGetLastError();
 }
 
-// A precomputed work list must cover the launch's grid (plan_rows >= its work entries).
-static hipError_t check_plan(const int32_t* plan, int64_t plan_rows, const Layout& L) {
+// A precomputed work list must cover the grid it is made for.
+static hipError_t check_plan(const int32_t* plan, int64_t plan_rows, int32_t batch, int32_t hq,
+                             int32_t hkv) {
     IE_REQUIRE(plan != nullptr, "null plan");
-    IE_REQUIRE(plan_rows >= L.nwork,
+    IE_REQUIRE(plan_rows >= ie_decode_attention_grid(batch, decode_units(hq, hkv)),
                "plan must hold ie_decode_attention_grid(batch, units) rows");
     IE_REQUIRE((reinterpret_cast<uintptr_t>(plan) & 15) == 0, "plan must be 16-byte aligned");
     return hipSuccess;
@@ -990,17 +922,20 @@ static hipError_t decode_plain(const ie_bf16* q, int64_t q_stride_b, int64_t q_s
                                const int32_t* num_decoding, float scale, ie_bf16* out,
                                int64_t out_stride_b, int64_t out_stride_h, void* workspace,
                                size_t workspace_bytes, const int32_t* plan, int64_t plan_rows,
-                               bool planned, hipStream_t stream) {
+                               bool planned, hipStream_t stream, size_t max_bytes = SIZE_MAX) {
     Layout L{};
     hipError_t e = check_decode(q, batch, num_q_heads, cache, cached_lens, slot_ids, num_decoding,
-                                out, q_stride_b, q_stride_h, workspace, workspace_bytes, &L);
+                                out, q_stride_b, q_stride_h, workspace, workspace_bytes, &L, true,
+                                max_bytes);
     if (e != hipSuccess || batch == 0) return e;
-    if (planned && (e = check_plan(plan, plan_rows, L)) != hipSuccess) return e;
+    if (planned && (e = check_plan(plan, plan_rows, batch, num_q_heads,
+                                   (int32_t)cache->num_kv_heads)) != hipSuccess)
+        return e;
     DecodeArgs a = decode_args(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens,
                                slot_ids, num_decoding, scale, out, out_stride_b, out_stride_h,
                                workspace, L);
     a.plan = planned ? plan : nullptr;
-    return decode_launch<false>(a, L, batch, cache, stream);
+    return decode_launch<false>(a, L, stream);
 }
 
 extern "C" hipError_t ie_decode_attention(
@@ -1040,7 +975,9 @@ static hipError_t decode_rope(
                                 false);
     if (e != hipSuccess || batch == 0) return e;
     IE_REQUIRE(k && v && q_norm_weight && k_norm_weight && cos && sin, "null pointer");
-    if (planned && (e = check_plan(plan, plan_rows, L)) != hipSuccess) return e;
+    if (planned && (e = check_plan(plan, plan_rows, batch, num_q_heads,
+                                   (int32_t)cache->num_kv_heads)) != hipSuccess)
+        return e;
     DecodeArgs a = decode_args(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens,
                                slot_ids, num_decoding, scale, out, out_stride_b, out_stride_h,
                                workspace, L);
@@ -1058,7 +995,7 @@ static hipError_t decode_rope(
     a.cos_sb = cos_stride_b;
     a.sin_sb = sin_stride_b;
     a.eps = eps;
-    return decode_launch<true>(a, L, batch, cache, stream);
+    return decode_launch<true>(a, L, stream);
 }
 
 extern "C" hipError_t ie_decode_attention_rope(
@@ -1190,8 +1127,7 @@ extern "C" hipError_t ie_decode_attention_noalloc(
     IE_REQUIRE(num_q_heads > 0 && num_q_heads % cache->num_kv_heads == 0 &&
                    num_q_heads / cache->num_kv_heads <= 16,
                "num_q_heads must be num_kv_heads times a GQA ratio of 1 to 16");
-    const Layout L =
-        workspace_layout(batch, num_q_heads, decode_units(num_q_heads, (int)cache->num_kv_heads));
+    const Layout L = call_layout(batch, num_q_heads, (int)cache->num_kv_heads, DA_SCRATCH_BYTES);
     IE_REQUIRE(batch <= DA_COUNT_CAP && num_q_heads <= DA_COUNT_HEADS &&
                    L.bytes <= DA_SCRATCH_BYTES,
                "batch too large for the no-alloc decode scratch (at most 1024 sequences and "
@@ -1199,7 +1135,7 @@ extern "C" hipError_t ie_decode_attention_noalloc(
     void* ws = nullptr;
     e = scratch_address(&ws);
     if (e != hipSuccess) return e;
-    return ie_decode_attention(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens,
-                               slot_ids, num_decoding, scale, out, out_stride_b, out_stride_h, ws,
-                               DA_SCRATCH_BYTES, stream);
+    return decode_plain(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens, slot_ids,
+                        num_decoding, scale, out, out_stride_b, out_stride_h, ws, DA_SCRATCH_BYTES,
+                        nullptr, 0, false, stream, DA_SCRATCH_BYTES);
 }

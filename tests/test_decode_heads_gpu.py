@@ -1,0 +1,99 @@
+"""The decode kernel's tiles at their edges: a wave's block holds 32 tokens, a workgroup round 32 per
+wave (4-, 2- and one-wave workgroups by batch), the 16 columns of a tile hold a KV head's query
+heads. Sequence lengths around those sizes at odd and full ratios, workgroups of every width, the
+few-KV-head layouts whose entries are cut to the workspace, `out` rows that take no 8-byte store, and
+V scales that leave the fp16 window mid-sequence; against the oracle with the bf16 tolerance."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_attn_close, bf16_np, cache_np, say
+from oracle import attention as oat
+
+pytestmark = pytest.mark.gpu
+SCALE = 128 ** -0.5
+EDGES = [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 160, 255, 257, 640, 1023, 4097]
+
+
+def _ref(wl):
+    return oat.decode_attention(bf16_np(wl.q), cache_np(wl.cache), wl.cached_lens.numpy(),
+                                wl.slot_ids.numpy(), int(wl.num_decoding[0]), SCALE)
+
+
+def _run(ie, wl, dev, out=None):
+    g = wl.to(dev)
+    out = ie.decode_attention(g.q, g.cache, g.cached_lens, g.slot_ids, g.num_decoding, SCALE,
+                              out=out)
+    torch.cuda.synchronize()
+    return bf16_np(out)
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (24, 8), (7, 1), (64, 4), (16, 2), (16, 1)])
+def test_lengths_at_tile_edges(ie, workloads, dev, hq, hkv):
+    say(f"decode edges {hq}/{hkv}")
+    wl = workloads.decode_workload(EDGES, seed=71, hq=hq, hkv=hkv)
+    assert_attn_close(_run(ie, wl, dev), _ref(wl), f"{hq}/{hkv}")
+
+
+@pytest.mark.parametrize("batch,hq,hkv", [(65, 16, 8), (129, 16, 8), (70, 64, 8), (140, 32, 8),
+                                          (300, 12, 4), (300, 64, 4)])
+def test_narrow_workgroups(ie, workloads, dev, batch, hq, hkv):
+    say(f"decode B={batch} {hq}/{hkv}")
+    ctx = [EDGES[i % 15] for i in range(batch)]
+    wl = workloads.decode_workload(ctx, seed=72, hq=hq, hkv=hkv)
+    assert_attn_close(_run(ie, wl, dev), _ref(wl), f"B={batch} {hq}/{hkv}")
+
+
+def test_out_rows_without_8_byte_alignment(ie, workloads, dev):
+    wl = workloads.decode_workload([33, 2000, 700], seed=73, hq=32, hkv=8)
+    buf = torch.full((3, 32, 131), 5.0, dtype=torch.bfloat16, device=dev)
+    out = buf[:, :, 1:129]
+    assert_attn_close(_run(ie, wl, dev, out), _ref(wl), "odd out rows")
+    assert (buf[:, :, 0] == 5.0).all() and (buf[:, :, 129:] == 5.0).all()
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (32, 8)])
+def test_v_scales_that_move(ie, workloads, dev, hq, hkv):
+    """V's scales rise by 2^12 and fall by 2^14 along the sequence (the exponent under which P times
+    scale is held in fp16 has to follow): outputs relative to the largest of them."""
+    wl = workloads.decode_workload([1500, 90, 3000], seed=74, hq=hq, hkv=hkv)
+    vs = wl.cache.v_scale
+    vs[:, :, 200:700] *= 2.0 ** 12
+    vs[:, :, 700:] *= 2.0 ** -2
+    got, ref = _run(ie, wl, dev), _ref(wl)
+    scale = np.abs(ref).max(axis=-1, keepdims=True)
+    assert_attn_close(got / scale, ref / scale, "moving V scales", rel=False)
+
+
+def test_fused_form_many_heads_one_wave_workgroups(ie, dev):
+    """decode_attention_rope where q's rows lie over the second stage (ratio 16, one wave per
+    workgroup): the same outputs as fused_rope_kv_decode then decode_attention, bit for bit in the
+    cache, within the tolerance in the output (the new token enters from registers)."""
+    hq, hkv, B, L = 64, 4, 520, 400
+    g = torch.Generator().manual_seed(75)
+    qkv = torch.randn(B, (hq + 2 * hkv) * 128, generator=g).bfloat16().to(dev)
+    q, k, v = (x.view(B, -1, 128) for x in qkv.split([hq * 128, hkv * 128, hkv * 128], -1))
+    w = (1 + 0.2 * torch.randn(2, 128, generator=g)).bfloat16().to(dev)
+    lens = torch.randint(0, L - 1, (B,), generator=g, dtype=torch.int32).to(dev)
+    slots = torch.randperm(B, generator=g).int().to(dev)
+    ang = lens[:, None, None].float() * (1e6 ** (-torch.arange(0, 128, 2, device=dev) / 128.0))
+    cos, sin = ang.cos().bfloat16(), ang.sin().bfloat16()
+    nd = torch.tensor([B], dtype=torch.int32, device=dev)
+    caches = []
+    for _ in range(2):
+        c = ie.make_layer_cache(B, hkv, L, 128, device=dev)
+        gc = torch.Generator(device=dev).manual_seed(76)
+        c.k.copy_(torch.randint(-127, 128, c.k.shape, generator=gc, device=dev))
+        c.v.copy_(torch.randint(-127, 128, c.v.shape, generator=gc, device=dev))
+        c.k_scale.copy_(torch.rand(c.k_scale.shape, generator=gc, device=dev) * 0.02)
+        c.v_scale.copy_(torch.rand(c.v_scale.shape, generator=gc, device=dev) * 0.02)
+        caches.append(c)
+    out = ie.decode_attention_rope(q, k, v, w[0], w[1], cos, sin, slots, caches[0], lens, nd, 1e-6,
+                                   SCALE)
+    qn = ie.fused_rope_kv_decode(q, k, v, w[0], w[1], cos, sin, slots, caches[1], lens, nd, 1e-6)
+    ref = ie.decode_attention(qn, caches[1], lens, slots, nd, SCALE)
+    torch.cuda.synchronize()
+    for name in ("k", "v", "k_scale", "v_scale"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
+    assert_attn_close(bf16_np(out), bf16_np(ref), "fused against two launches")
