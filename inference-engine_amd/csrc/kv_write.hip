@@ -3,6 +3,8 @@
 //   quantize_kv_prefill_kernel   prefill quantize-on-write (+ K calibration on a first chunk)
 //   kcal_max_kernel              first-chunk K calibration ahead of the quantize, long steps
 //   quantize_kv_stream_kernel    the quantize launch of long steps (resident grid, prefetch)
+//   norm_rope_rows_kernel        prefill q/k RMSNorm + RoPE of 16-byte aligned rows
+//   fused_norm_rope_prefill_kernel  the same for any alignment
 //   fused_rope_kv_decode_kernel  decode q/k RMSNorm + RoPE, q * calibration, K/V quantize
 //   dequantize_kv_prefix_kernel  int8 prefix -> bf16
 //
@@ -652,6 +654,110 @@ __global__ __launch_bounds__(256) void fused_norm_rope_prefill_kernel(
     }
 }
 
+// The same rows where they are 16-byte aligned (what an engine's packed rows are). What bounds it is HBM (each row read and written once); the kernel above moves two
+// bytes per lane and load, 128 bytes per instruction. Here a wave takes PP groups of four head rows
+// of one token: 16 lanes per row, lane c holding channels 8 c ... 8 c + 7 (one 16-byte load and
+// store), the second half of the row in lanes 8 ... 15, so the RoPE partner of a channel sits 8 lanes
+// away. Bit for bit the arithmetic above: the butterfly over 64 lanes becomes the same additions
+// across lanes (distance 32, 16, 8) and then inside them (4, 2, 1); each rstd is computed by one
+// lane of a row (lane p: group p's) and broadcast. 8,192 tokens of 16 + 8 heads: 25.9 -> 21.2 us
+// (4.86 TB/s; a large copy reaches 5.16), 12,288 42.0 -> 29.6, 64 tokens 4.1 -> 2.5.
+// grid (cdiv(N, 4), cdiv(groups, PP)), block 256: one wave per token.
+template <int CTRL>
+__device__ __forceinline__ float row_bcast(float x) {  // row_newbcast
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+struct NormRopeArgs {
+    const uint16_t *q, *k, *qw, *kw, *cos, *sin;
+    int64_t q_st, q_sh, k_st, k_sh, cos_st, sin_st;
+    uint16_t *qo, *ko;
+    int64_t qo_st, qo_sh, ko_st, ko_sh;
+    int64_t n;
+    int hq, rows;  // rows: query then key heads
+    float eps;
+};
+template <int PP>
+__global__ __launch_bounds__(256) void norm_rope_rows_kernel(NormRopeArgs a) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63, c = lane & 15, rr = lane >> 4;
+    const int64_t t = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (t >= a.n) return;
+    const int r0 = 4 * PP * blockIdx.y + rr;
+    auto unpack = [](uint4 v, float (&f)[8]) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f[2 * j] = bf16lo(w[j]);
+            f[2 * j + 1] = bf16hi(w[j]);
+        }
+    };
+    uint4 x[PP];
+#pragma unroll
+    for (int p = 0; p < PP; ++p) {
+        const int r = r0 + 4 * p;
+        x[p] = make_uint4(0u, 0u, 0u, 0u);
+        if (r < a.rows)
+            x[p] = *reinterpret_cast<const uint4*>(
+                (r < a.hq ? a.q + t * a.q_st + r * a.q_sh : a.k + t * a.k_st + (r - a.hq) * a.k_sh) +
+                8 * c);
+    }
+    const uint4 cv = *reinterpret_cast<const uint4*>(a.cos + t * a.cos_st + 8 * (c & 7));
+    const uint4 sv = *reinterpret_cast<const uint4*>(a.sin + t * a.sin_st + 8 * (c & 7));
+    const uint4 qv = *reinterpret_cast<const uint4*>(a.qw + 8 * c);
+    const uint4 kv = *reinterpret_cast<const uint4*>(a.kw + 8 * c);
+    float my_ss = 0.f;  // lane p of a row (and p + 8): the sum of squares of group p's row
+#pragma unroll
+    for (int p = 0; p < PP; ++p) {
+        float f[8];
+        unpack(x[p], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float s = f[j] * f[j];
+            s = s + dpp<DPP_HALF_MIRROR>(dpp<DPP_XOR3>(s));  // channel distance 32: lane ^ 4
+            s = s + dpp<DPP_XOR2>(s);
+            f[j] = s + dpp<DPP_XOR1>(s);
+        }
+        float s[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = f[j] + f[j + 4];
+        const float half = (s[0] + s[2]) + (s[1] + s[3]);
+        const float ss = half + dpp<DPP_ROR8>(half);
+        my_ss = (c & 7) == p ? ss : my_ss;
+    }
+    const float my_rstd = row_rstd(my_ss, a.eps);
+    float cs[8], sn[8], wq[8], wk[8];
+    unpack(cv, cs);
+    unpack(sv, sn);
+    unpack(qv, wq);
+    unpack(kv, wk);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sn[j] = c < 8 ? -sn[j] : sn[j];
+#pragma unroll
+    for (int p = 0; p < PP; ++p) {
+        const int r = r0 + 4 * p;
+        const bool is_q = r < a.hq;
+        const float rstd = p == 0   ? row_bcast<0x150>(my_rstd)
+                           : p == 1 ? row_bcast<0x151>(my_rstd)
+                           : p == 2 ? row_bcast<0x152>(my_rstd)
+                           : p == 3 ? row_bcast<0x153>(my_rstd)
+                           : p == 4 ? row_bcast<0x154>(my_rstd)
+                                    : row_bcast<0x155>(my_rstd);
+        float f[8];
+        unpack(x[p], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = (f[j] * rstd) * (is_q ? wq[j] : wk[j]);
+        float o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = (f[j] * cs[j]) + (dpp<DPP_ROR8>(f[j]) * sn[j]);
+        if (r < a.rows)
+            *reinterpret_cast<uint4*>((is_q ? a.qo + t * a.qo_st + r * a.qo_sh
+                                            : a.ko + t * a.ko_st + (r - a.hq) * a.ko_sh) +
+                                      8 * c) =
+                make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]),
+                           pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
+    }
+}
+
 constexpr int DQ_TOKENS = 64;
 
 // grid (num_entries, Hkv, ceil(max_len / 64)), block 256 (kernels.py:868-932): 16 lanes x 8
@@ -696,6 +802,16 @@ __global__ __launch_bounds__(256) void dequantize_kv_prefix_kernel(
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Row groups per wave of norm_rope_rows_kernel: one while the step is small (latency: 64 tokens of
+// 16 + 8 heads 2.5 us, against 4.2 with six; 1,054 tokens 5.2 against 6.3), six or three from about
+// 4,096 such tokens (the token's cos and sin and the weights are read once per wave: 12,288 tokens
+// 29.6 us against 34.6 with one).
+static int nr_groups(int64_t tokens, int rows) {
+    const int groups = (rows + 3) / 4;
+    if (tokens * rows < 4096 * 24 || groups < 3) return 1;
+    return groups % 6 == 0 || groups >= 12 ? 6 : 3;
+}
 
 }  // namespace ie
 
@@ -791,6 +907,32 @@ extern "C" hipError_t ie_fused_norm_rope_prefill(
                "null pointer");
     IE_REQUIRE(num_tokens < (1LL << 31), "too many tokens");
     const int rows = num_q_heads + num_kv_heads;
+    const int64_t strides = q_stride_tok | q_stride_head | k_stride_tok | k_stride_head |
+                            cos_stride_tok | sin_stride_tok | q_out_stride_tok |
+                            q_out_stride_head | k_out_stride_tok | k_out_stride_head;
+    // (a few tokens of at most four rows finish sooner with a wave per row: 16 tokens of 2 + 1 heads
+    // 2.3 against 2.4 us, 1,054 tokens 3.1 against 2.8)
+    if (!(rows <= 4 && num_tokens <= 512) && strides % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(q_norm_weight) &&
+        aligned16(k_norm_weight) && aligned16(cos) && aligned16(sin) && aligned16(q_out) &&
+        aligned16(k_out)) {
+        NormRopeArgs a{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)q_norm_weight,
+                       (const uint16_t*)k_norm_weight, (const uint16_t*)cos, (const uint16_t*)sin,
+                       q_stride_tok, q_stride_head, k_stride_tok, k_stride_head, cos_stride_tok,
+                       sin_stride_tok, (uint16_t*)q_out, (uint16_t*)k_out, q_out_stride_tok,
+                       q_out_stride_head, k_out_stride_tok, k_out_stride_head, num_tokens,
+                       num_q_heads, rows, eps};
+        const int groups = (rows + 3) / 4;
+        const unsigned gx = (unsigned)((num_tokens + 3) / 4);
+        auto gy = [&](int pp) { return (unsigned)((groups + pp - 1) / pp); };
+        const int pp = nr_groups(num_tokens, rows);
+        if (pp == 6)
+            hipLaunchKernelGGL(norm_rope_rows_kernel<6>, dim3(gx, gy(6)), dim3(256), 0, stream, a);
+        else if (pp == 3)
+            hipLaunchKernelGGL(norm_rope_rows_kernel<3>, dim3(gx, gy(3)), dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL(norm_rope_rows_kernel<1>, dim3(gx, gy(1)), dim3(256), 0, stream, a);
+        return hipGetLastError();
+    }
     dim3 grid((unsigned)num_tokens, (unsigned)((rows + NR_ROWS_PER_WG - 1) / NR_ROWS_PER_WG));
     hipLaunchKernelGGL(fused_norm_rope_prefill_kernel, grid, dim3(256), 0, stream,
                        (const uint16_t*)q, q_stride_tok, q_stride_head, (const uint16_t*)k,

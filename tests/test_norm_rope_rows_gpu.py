@@ -1,0 +1,33 @@
+"""fused_norm_rope_prefill on 16-byte aligned rows (16 lanes per head row) against the form for any
+alignment (one wave per row group, the one the oracle tests pin as well), bit for bit: head counts
+that fill a wave's row groups, leave a remainder or mix q and k in a group, token counts around the
+groups-per-wave rule, rows of very different magnitude, and rows of zeros."""
+
+import pytest
+import torch
+
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (2, 1), (7, 7), (5, 1), (40, 8), (1, 1)])
+@pytest.mark.parametrize("n", [1, 3, 515, 4097])
+def test_aligned_rows_equal_unaligned_rows(ie, dev, hq, hkv, n):
+    say(f"norm rope {hq}+{hkv} heads, {n} tokens")
+    g = torch.Generator(device=dev).manual_seed(81)
+    h = hq + hkv
+    x = torch.randn(n, h, 128, generator=g, device=dev)
+    x *= 10.0 ** torch.randint(-6, 6, (n, h, 1), generator=g, device=dev)
+    x[n // 2, h - 1] = 0.0
+    x = x.bfloat16()
+    w = (1 + 0.3 * torch.randn(2, 128, generator=g, device=dev)).bfloat16()
+    ang = 1000 * torch.rand(n, 1, 64, generator=g, device=dev)
+    cos, sin = ang.cos().bfloat16(), ang.sin().bfloat16()
+    wide = torch.empty(n, h * 128 + 3, dtype=torch.bfloat16, device=dev)  # rows 2 bytes off
+    odd = wide[:, 1:h * 128 + 1].view(n, h, 128).copy_(x)
+    got = ie.fused_norm_rope_prefill(x[:, :hq], x[:, hq:], w[0], w[1], cos, sin, 1e-6)
+    ref = ie.fused_norm_rope_prefill(odd[:, :hq], odd[:, hq:], w[0], w[1], cos, sin, 1e-6)
+    torch.cuda.synchronize()
+    for a, b in zip(got, ref):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
