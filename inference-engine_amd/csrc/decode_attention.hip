@@ -187,7 +187,6 @@ struct DecodeArgs {
     float eps;
 };
 
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -202,22 +201,7 @@ constexpr float DA_SLACK = 3.0f;  // the running max moves when a score exceeds 
 constexpr int DA_VE_TOP = 12, DA_VE_WIN = 7;
 static_assert(16 * DA_OROW * 4 <= 2 * DA_STAGE, "a wave's output overlays its stages");
 
-// 16 (4) bytes per lane from memory to LDS at lds + 16 (4) lane, counted by vmcnt; lanes past the
-// descriptor's range touch no memory. In assembly so that the compiler's own waits do not drain
-// the stages in flight: the waits are the caller's. s_nop: m0 is read by the load.
-__device__ __forceinline__ void da_dma16(v4u rsrc, int off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
-                 :: "s"(lds), "v"(off), "s"(rsrc) : "memory", "m0");
-}
-__device__ __forceinline__ void da_dma4(const float* p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                 :: "s"(lds), "v"(p) : "memory", "m0");
-}
-constexpr int DA_DMAS = 9;  // per block: 4 K, 4 V, the scales
-__device__ __forceinline__ v4u da_rsrc(const void* base, uint32_t bytes) {
-    const uint64_t p = (uint64_t)base;
-    return v4u{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, (uint32_t)RSRC_WORD3};
-}
+constexpr int DA_DMAS = 9;  // loads per block: 4 K, 4 V, the scales
 
 // eight int8 (two words) -> fp16, exactly
 __device__ __forceinline__ half8_t da_cvt8(uint32_t x0, uint32_t x1) {
@@ -392,25 +376,24 @@ decode_attention_kernel(DecodeArgs a) {
     const int slot = b < 64 ? __builtin_amdgcn_readlane(slot0, b) : uniform(a.slot_ids[b]);
     const int t_begin = split * piece, t_end = min(t_begin + piece, n_end);
 
-    const v4u rk = da_rsrc(a.c.k + slot * a.c.stride_slot + hk * a.c.stride_head,
+    const v4u rk = rsrc_words(a.c.k + slot * a.c.stride_slot + hk * a.c.stride_head,
                            (uint32_t)t_end * DA_D);
-    const v4u rv = da_rsrc(a.c.v + slot * a.c.stride_slot + hk * a.c.stride_head,
+    const v4u rv = rsrc_words(a.c.v + slot * a.c.stride_slot + hk * a.c.stride_head,
                            (uint32_t)t_end * DA_D);
     // lanes 0 ... 31: the block's K scales, lanes 32 ... 63 its V scales
     const float* sc = (lane < DA_TOK ? a.c.k_scale : a.c.v_scale) +
                       slot * a.c.scale_stride_slot + hk * a.c.scale_stride_head;
     uint8_t* ring = s_ring[wave][0];
-    const uint32_t lds0 = (uint32_t)uniform(
-        (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)ring);
+    const uint32_t lds0 = lds_addr(ring);
     const int koff = (lane >> 3) * DA_D + (((lane & 7) ^ (lane >> 3)) << 4), voff = 16 * lane;
     auto issue = [&](int stage, int t0) {
         const uint32_t l = lds0 + stage * DA_STAGE;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) da_dma16(rk, t0 * DA_D + 1024 * i + koff, l + 1024 * i);
-        da_dma4(sc + min(t0 + (lane & (DA_TOK - 1)), t_end - 1), l + DA_SC);
+        for (int i = 0; i < 4; ++i) dma16<true>(rk, t0 * DA_D + 1024 * i + koff, l + 1024 * i);
+        dma4(sc + min(t0 + (lane & (DA_TOK - 1)), t_end - 1), l + DA_SC);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            da_dma16(rv, t0 * DA_D + 1024 * i + voff, l + DA_V + 1024 * i);
+            dma16<true>(rv, t0 * DA_D + 1024 * i + voff, l + DA_V + 1024 * i);
     };
     // this wave's blocks: w, w + W, ... of the piece's 32-token blocks
     const int nb = (t_end - t_begin + DA_TOK - 1) / DA_TOK;
@@ -504,7 +487,7 @@ decode_attention_kernel(DecodeArgs a) {
         qraw[2] = *reinterpret_cast<const uint4*>(qp + 64);
         qraw[3] = *reinterpret_cast<const uint4*>(qp + 72);
         if (q_over && cw > 1) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            lds_reads_done();
             issue(1, t_first + W * DA_TOK);
         }
     } else {
@@ -545,8 +528,8 @@ decode_attention_kernel(DecodeArgs a) {
     s.vlo = (uint32_t)(DA_VE_TOP - DA_VE_WIN + 127) << 23;
     for (int j = 0, t0 = t_first; j < cw; ++j, t0 += W * DA_TOK) {
         // block j is here once at most block j + 1's loads (if any) are outstanding
-        if (j + 1 < cw) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(DA_DMAS) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (j + 1 < cw) wait_vm<DA_DMAS>();
+        else wait_vm<0>();
         uint8_t* st = ring + (j & 1) * DA_STAGE;
         if (t0 + DA_TOK <= t_end && !(kv_wave && j == cw - 1)) {
             da_block<false>(s, qf, kmul, st, t0, t_end, l16, g);
@@ -562,12 +545,12 @@ decode_attention_kernel(DecodeArgs a) {
                     reinterpret_cast<float*>(st + DA_SC)[t] = nks;
                     reinterpret_cast<float*>(st + DA_SC)[DA_TOK + t] = nvs;
                 }
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                lds_reads_done();
             }
             da_block<true>(s, qf, kmul, st, t0, t_end, l16, g);
         }
         if (j + 2 < cw) {  // every read of this stage has its data
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            lds_reads_done();
             issue(j & 1, t0 + 2 * W * DA_TOK);
         }
     }

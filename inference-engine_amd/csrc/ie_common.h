@@ -170,6 +170,40 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, RSRC_WORD3);
 }
 
+// Loads from memory straight into LDS: 16 (4) bytes per lane, landing at lds + 16 (4) lane, whatever
+// the lanes' addresses; counted by vmcnt, no registers held, lanes past a descriptor's range touch no
+// memory (their LDS bytes are undefined). In assembly: through the builtins the compiler drains every
+// such load in flight before the first LDS read that may alias, so the waits are the caller's
+// (wait_vm), and so is the order (lds_reads_done before a place is loaded over). s_nop: m0 is read by
+// the load.
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+template <bool NT>
+__device__ __forceinline__ void dma16(v4u rsrc, int off, uint32_t lds) {
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                     :: "s"(lds), "v"(off), "s"(rsrc) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :: "s"(lds), "v"(off), "s"(rsrc) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(const float* p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+                 :: "s"(lds), "v"(p) : "memory", "m0");
+}
+// The descriptor of make_rsrc as the four words the assembly takes (wave-uniform).
+__device__ __forceinline__ v4u rsrc_words(const void* base, uint32_t bytes) {
+    const uint64_t p = (uint64_t)base;
+    return v4u{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, (uint32_t)RSRC_WORD3};
+}
+// The LDS byte address of a __shared__ object.
+__device__ __forceinline__ uint32_t lds_addr(void* p) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p);
+}
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // ---------------------------------------------------------------------------------------------
 // Device-coherent accesses, for partial results that one workgroup writes and another merges in
 // the same launch: loads and stores with the device scope bit (sc1), served at the level all

@@ -81,13 +81,16 @@ constexpr int SG_MAX_TILES = 6;  // weight + x tiles, at most (LDS: 8 waves x 16
 // 32 S + 8 g .. + 8), loaded straight into registers like a swizzled weight; YFRAG (paired
 // gate/up form): y is written in that order, for a next GEMM that takes it as XFRAG (the MLP's
 // down projection), rows past M not written.
+// DMA (with HALF): the batches go straight to LDS (dma16), three or four of them in flight per wave
+// with no registers held and no store to LDS; the same fragments in the same order.
 // AMAX (with LOOP and XREG: the LM head): also the greedy token of every row, the first column
 // of the largest bf16 output (sample's greedy rule at tau = 0: larger value, then smaller index;
 // NaN never chosen): each lane keeps its best over its blocks, each workgroup folds its lanes'
 // and counts itself into a device-scope 64-bit max per row, and the last workgroup to finish
 // writes the tokens, clears the maxima and advances the sampler's seed.
 enum : int { SG_PLAIN = 0, SG_HALF = 1, SG_GLU = 2, SG_NORM = 4, SG_RES = 8, SG_SWZ = 16,
-             SG_LOOP = 32, SG_XREG = 64, SG_XFRAG = 128, SG_YFRAG = 256, SG_AMAX = 512 };
+             SG_LOOP = 32, SG_XREG = 64, SG_XFRAG = 128, SG_YFRAG = 256, SG_AMAX = 512,
+             SG_DMA = 1024 };
 
 // AMAX's outputs: per-row maxima keys[M] and a count (zero on entry, left zero), tokens (int64,
 // stride os) and the sampler's seed.
@@ -113,10 +116,20 @@ __device__ __forceinline__ uint64_t amax_key(float v, int i) {
 }
 constexpr int SG_XREG_K = SG_WAVES * 4 * SG_BK;  // the one K of the XREG form: 4 batches a wave
 
-template <int TT, int MT, int PT>
+// DMA: a wave's stage holds one batch: 8 weight rows and 16 MT rows of x, 128 bytes each, 16-byte
+// chunk c of row r at place c ^ (r & 7); as many stages as SG_DMA_LDS holds, at most four.
+constexpr int SG_DMA_LDS = 152 * 1024;
+template <int MT>
+struct SgStage {
+    static constexpr int W_BYTES = 1024, BYTES = W_BYTES + 2048 * MT;
+    static constexpr int FIT = SG_DMA_LDS / (SG_WAVES * BYTES), STAGES = FIT < 4 ? FIT : 4;
+    static constexpr int LOADS = BYTES / 1024;  // per wave and batch
+    static_assert(STAGES >= 2, "a stage in flight beside the one being read");
+};
+template <int TT, int MT, int PT, int RING = 0>
 struct SgLds {
     union {
-        uint8_t t[SG_WAVES][16 * TT * SG_LROW];          // per-wave transpose regions
+        uint8_t t[SG_WAVES][RING ? RING : 16 * TT * SG_LROW];  // per-wave transpose regions / stages
         sg_f32x4 acc[SG_WAVES][PT * MT][IE_WAVE];       // partial D tiles (after the loop)
     };
     float ss[SG_WAVES][16 * MT];  // NORM: each wave's sums of squares of x rows over its K slice
@@ -133,7 +146,9 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
     constexpr bool HALF = MODE & SG_HALF, GLU = MODE & SG_GLU, NORM = MODE & SG_NORM,
                    RES = MODE & SG_RES, SWZ = MODE & SG_SWZ, LOOP = MODE & SG_LOOP,
                    XREG = MODE & SG_XREG, XFRAG = MODE & SG_XFRAG, YFRAG = MODE & SG_YFRAG,
-                   AMAX = MODE & SG_AMAX;
+                   AMAX = MODE & SG_AMAX, DMA = MODE & SG_DMA;
+    static_assert(!DMA || (HALF && !XFRAG), "global -> LDS stages: 8-row tiles, row-major x");
+    using Stage = SgStage<MT>;
     constexpr bool PAIR = GLU && SWZ;  // gate and up rows paired inside each 16-row tile
     constexpr int WT = GLU && !PAIR ? 2 * NT : NT;  // weight tiles (GLU: NT gate, then NT up)
     static_assert(WT + MT <= SG_MAX_TILES, "LDS transpose region too large");
@@ -183,12 +198,13 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
                     continue;
                 }
                 const int row = 16 * (i < WT ? i % NT : i - WT) + 8 * h + lr;
-                loff[i][h] = (row * (int)(i < WT ? ws : xs) + k_begin + 8 * lc) * 2;
+                loff[i][h] = (row * (int)(i < WT ? ws : xs) + k_begin + 8 * (DMA ? lc ^ lr : lc)) * 2;
             }
     };
     int blk = blockIdx.x;
     setup(blk);
-    __shared__ __attribute__((aligned(16))) SgLds<TILES - T0, MT, NT> lds;
+    __shared__ __attribute__((aligned(16)))
+    SgLds<TILES - T0, MT, NT, DMA ? Stage::STAGES * Stage::BYTES : 0> lds;
     // XREG: the MFMA B fragments of x over the wave's slice, xf[b][t][mt] = x row 16 mt + l16,
     // k = 64 b + 32 t + 8 g .. + 8 of the slice (rows past M read zeros)
     typedef sg_bf16x8 XFrag[2][MT];
@@ -315,7 +331,7 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
     // join, and left alone the scheduler sinks them below the MFMAs.
     const int nb = (kw + SG_BK - 1) / SG_BK;
     Batch ra, rb, rc, rd;  // rc, rd: XREG only
-    load(ra, 0);
+    if constexpr (!DMA) load(ra, 0);
     if constexpr (XREG) {  // a ring of four batches, three in flight ahead of the MFMAs
         load(rb, 1);
         load(rc, 2);
@@ -343,6 +359,60 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
         load(rc, 2, more);
         __builtin_amdgcn_sched_barrier(0);
         compute(rd, xf[3]);
+    } else if constexpr (DMA) {  // kw a multiple of 64
+        const v4u dw = rsrc_words(w + (int64_t)n0 * ws, (uint32_t)(WROWS * ws * 2));
+        const v4u dx = rsrc_words(x, (uint32_t)(M * xs * 2));
+        const uint32_t lds0 = lds_addr(reg);
+        auto issue = [&](int b) {
+            const uint32_t st = lds0 + (b % Stage::STAGES) * Stage::BYTES;
+            dma16<true>(dw, loff[0][0] + 128 * b, st);
+#pragma unroll
+            for (int i = 0; i < 2 * MT; ++i)
+                dma16<false>(dx, loff[1 + i / 2][i % 2] + 128 * b, st + Stage::W_BYTES + 1024 * i);
+        };
+#pragma unroll
+        for (int b = 0; b < Stage::STAGES; ++b)
+            if (b < nb) issue(b);
+        for (int b = 0; b < nb; ++b) {
+            // batch b is here once only the batches after it are outstanding
+            const int ahead = min(Stage::STAGES - 1, nb - 1 - b);
+            if (ahead == 3) wait_vm<3 * Stage::LOADS>();
+            else if (ahead == 2) wait_vm<2 * Stage::LOADS>();
+            else if (ahead == 1) wait_vm<Stage::LOADS>();
+            else wait_vm<0>();
+            const uint8_t* st = reg + (b % Stage::STAGES) * Stage::BYTES;
+            sg_bf16x8 f[2][TILES];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < TILES; ++i) {
+                    // rows 8..15 of the weight tile repeat rows 0..7 (their outputs are not stored)
+                    f[t][i] = *reinterpret_cast<const sg_bf16x8*>(
+                        st + (i == 0 ? 128 * (l16 & 7)
+                                     : Stage::W_BYTES + 2048 * (i - 1) + 128 * l16) +
+                        16 * ((4 * t + g) ^ (l16 & 7)));
+                }
+            if (b + Stage::STAGES < nb) {  // the batch's place is free once its reads are done
+                lds_reads_done();
+                issue(b + Stage::STAGES);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[0][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[t][0], f[t][1 + mt],
+                                                                         acc[0][mt], 0, 0, 0);
+                if (NORM) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                        for (int j = 0; j < 8; j += 2) {
+                            const sg_bf16x2 p = {f[t][1 + mt][j], f[t][1 + mt][j + 1]};
+                            ss[mt] = __builtin_amdgcn_fdot2_f32_bf16(p, p, ss[mt], false);
+                        }
+                }
+            }
+        }
     } else {
         for (int b = 0; b < nb; b += 2) {
             load(rb, b + 1);
@@ -550,6 +620,16 @@ struct SgCall {
 
 template <int MT, int NT, int MODE>
 void sg_go(dim3 grid, hipStream_t s, const SgCall& c) {
+    // 8-row tiles of at most one workgroup per CU through LDS stages (the same bits). Measured on
+    // weights from HBM, 1 / 16 / 32 / 64 rows: [2048, 6144] 8.4 / 10.0 / 11.8 / 17.4 -> 7.1 / 10.0 /
+    // 11.6 / 16.9 us, [2048, 2048] 4.0 / 4.6 / 5.3 / 7.6 -> 3.8 / 4.5 / 5.15 / 7.2. With more
+    // workgroups than CUs the stages' LDS keeps a second one off the CU ([12288, 2048] 13.1 -> 16.7).
+    if constexpr ((MODE & SG_HALF) && !(MODE & (SG_XFRAG | SG_DMA))) {
+        if (c.k % (SG_WAVES * SG_BK) == 0 && (int)grid.x <= device_cu_count()) {
+            sg_go<MT, NT, MODE | SG_DMA>(grid, s, c);
+            return;
+        }
+    }
     hipLaunchKernelGGL((skinny_gemm_kernel<MT, NT, MODE>), grid, dim3(SG_THREADS), 0, s, c.x,
                        c.xs, c.m, c.w, c.ws, c.k, c.y, c.ys, c.nh, c.eps,
                        c.nblk > 0 ? c.nblk : (int)grid.x, c.am);
