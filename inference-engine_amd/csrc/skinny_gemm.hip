@@ -81,6 +81,8 @@ constexpr int SG_MAX_TILES = 6;  // weight + x tiles, at most (LDS: 8 waves x 16
 // 32 S + 8 g .. + 8), loaded straight into registers like a swizzled weight; YFRAG (paired
 // gate/up form): y is written in that order, for a next GEMM that takes it as XFRAG (the MLP's
 // down projection), rows past M not written.
+// RPAIR (with GLU, row-major): the paired tiles of SWZ's gate/up order read from the row-major
+// weight (half a tile's rows from the gate part, half from the up part), 8 NT columns per workgroup.
 // DMA (with HALF): the batches go straight to LDS (dma16), three or four of them in flight per wave
 // with no registers held and no store to LDS; the same fragments in the same order.
 // AMAX (with LOOP and XREG: the LM head): also the greedy token of every row, the first column
@@ -90,7 +92,7 @@ constexpr int SG_MAX_TILES = 6;  // weight + x tiles, at most (LDS: 8 waves x 16
 // writes the tokens, clears the maxima and advances the sampler's seed.
 enum : int { SG_PLAIN = 0, SG_HALF = 1, SG_GLU = 2, SG_NORM = 4, SG_RES = 8, SG_SWZ = 16,
              SG_LOOP = 32, SG_XREG = 64, SG_XFRAG = 128, SG_YFRAG = 256, SG_AMAX = 512,
-             SG_DMA = 1024 };
+             SG_DMA = 1024, SG_RPAIR = 2048 };
 
 // AMAX's outputs: per-row maxima keys[M] and a count (zero on entry, left zero), tokens (int64,
 // stride os) and the sampler's seed.
@@ -146,14 +148,15 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
     constexpr bool HALF = MODE & SG_HALF, GLU = MODE & SG_GLU, NORM = MODE & SG_NORM,
                    RES = MODE & SG_RES, SWZ = MODE & SG_SWZ, LOOP = MODE & SG_LOOP,
                    XREG = MODE & SG_XREG, XFRAG = MODE & SG_XFRAG, YFRAG = MODE & SG_YFRAG,
-                   AMAX = MODE & SG_AMAX, DMA = MODE & SG_DMA;
+                   AMAX = MODE & SG_AMAX, DMA = MODE & SG_DMA, RPAIR = MODE & SG_RPAIR;
     static_assert(!DMA || (HALF && !XFRAG), "global -> LDS stages: 8-row tiles, row-major x");
     using Stage = SgStage<MT>;
-    constexpr bool PAIR = GLU && SWZ;  // gate and up rows paired inside each 16-row tile
+    constexpr bool PAIR = GLU && (SWZ || RPAIR);  // gate and up rows paired inside each 16-row tile
     constexpr int WT = GLU && !PAIR ? 2 * NT : NT;  // weight tiles (GLU: NT gate, then NT up)
     static_assert(WT + MT <= SG_MAX_TILES, "LDS transpose region too large");
     static_assert(!HALF || NT == 1, "8-row n-tiles come one per workgroup");
-    static_assert(!GLU || SWZ || NT * MT <= SG_WAVES, "GLU: at most one output tile per wave");
+    static_assert(!GLU || PAIR || NT * MT <= SG_WAVES, "GLU: at most one output tile per wave");
+    static_assert(!RPAIR || (GLU && !SWZ && !HALF), "paired rows of a row-major gate/up weight");
     static_assert(!(SWZ && HALF), "the fragment-ordered weight comes in 16-row groups");
     static_assert(!LOOP || !(GLU || RES || HALF || (NORM && !XREG)),
                   "the looping grid: plain launches (NORM: with x in registers)");
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
     float abv = -INFINITY;  // AMAX: this lane's best output so far, and its column
     int abi = 0x7fffffff;
     constexpr int XNB = XREG ? SG_XREG_K / SG_WAVES / SG_BK : 1;  // batches of x held per wave
-    constexpr int WROWS = HALF ? 8 : 16 * NT;  // weight rows per workgroup (per half in GLU)
+    constexpr int WROWS = HALF ? 8 : RPAIR ? 8 * NT : 16 * NT;  // weight rows per workgroup (per half in GLU)
     constexpr int TILES = WT + MT;  // W tiles 0..WT-1, then x tiles
     constexpr int T0 = SWZ ? WT : 0;  // the first tile that goes through LDS (its LDS row: 16 (i - T0))
     const int tid = threadIdx.x, lane = tid & 63;
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
                   k_begin = (int)(XREG ? wave : (wave + bk) % SG_WAVES) * kw;
         kstep0 = k_begin / 32;
         rw = make_rsrc(w + (int64_t)n0 * ws, (uint32_t)(WROWS * ws * 2));
-        ru = make_rsrc(w + ((int64_t)nh + n0) * ws, (uint32_t)(GLU && !PAIR ? WROWS * ws * 2 : 0));
+        ru = make_rsrc(w + ((int64_t)nh + n0) * ws, (uint32_t)(GLU && !SWZ ? WROWS * ws * 2 : 0));
 #pragma unroll
         for (int i = 0; i < TILES; ++i)
 #pragma unroll
@@ -197,7 +200,9 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
                     loff[i][h] = ((k_begin / 32 + h) * NT + i % NT) * 1024 + 16 * lane;
                     continue;
                 }
-                const int row = 16 * (i < WT ? i % NT : i - WT) + 8 * h + lr;
+                // RPAIR: half h of tile i is rows 8 i .. + 7 of the gate (h = 0) or up (h = 1) part
+                const int row = RPAIR && i < WT ? 8 * i + lr
+                                                : 16 * (i < WT ? i % NT : i - WT) + 8 * h + lr;
                 loff[i][h] = (row * (int)(i < WT ? ws : xs) + k_begin + 8 * (DMA ? lc ^ lr : lc)) * 2;
             }
     };
@@ -276,7 +281,8 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
                 }
                 if (i < WT)
                     r[i][h] = __builtin_amdgcn_raw_buffer_load_b128(
-                        i < NT ? rw : ru, in ? loff[i][h] + 128 * b : -1, 0, IE_SKINNY_W_AUX);
+                        (RPAIR ? h == 0 : i < NT) ? rw : ru, in ? loff[i][h] + 128 * b : -1, 0,
+                        IE_SKINNY_W_AUX);
                 else if (XFRAG)  // 32-column step h of the batch, m-tile i - WT: one 1 KB block
                     r[i][h] = __builtin_amdgcn_raw_buffer_load_b128(
                         rx,
@@ -453,7 +459,11 @@ __global__ __launch_bounds__(SG_THREADS) void skinny_gemm_kernel(
                 lds.acc[wave][nt * MT + mt][lane] = acc[round * NT + nt][mt];
         __syncthreads();
         for (int tile = wave; tile < NT * MT; tile += SG_WAVES) {
-            const int rot = XREG ? blk % SG_WAVES : 0;
+            // RPAIR: the order in which the separate-tile form of nblk-column workgroups adds, in
+            // which position v holds slice (v + column / nblk) mod 8; wave u holds slice u + blk
+            const int rot = XREG    ? blk % SG_WAVES
+                            : RPAIR ? (8 * (blk * NT + tile / MT) / nblk - blk) & (SG_WAVES - 1)
+                                    : 0;
             sg_f32x4 t = lds.acc[rot][tile][lane];
 #pragma unroll
             for (int v = 1; v < SG_WAVES; ++v) t += lds.acc[(v + rot) % SG_WAVES][tile][lane];
@@ -703,6 +713,25 @@ void sg_glu_mt(int mt, int n_tiles, dim3 grid, hipStream_t s, const SgCall& c) {
     }
 }
 
+// The row-major gate/up weight in paired tiles, three per workgroup (24 columns): where the busiest
+// CU then has fewer columns to do than in 16 n_tiles-column workgroups, every CU working (6,144
+// columns: 256 workgroups of 24, against 192 of 32 or 384 of 16). The same bits.
+// Measured at [12288, 2048], 1 / 16 / 32 / 48 rows: 12.5 / 12.8 / 14.3 / 18.6 -> 11.5 / 11.5 / 12.7 /
+// 14.4 us.
+bool sg_row_pairs(int cols, int n_tiles, int mt) {
+    const int cus = device_cu_count();
+    auto most = [&](int per) { return (cols / per + cus - 1) / cus * per; };
+    return cols % 24 == 0 && 3 + mt <= SG_MAX_TILES && most(24) < most(16 * n_tiles);
+}
+template <int EXTRA>
+void sg_row_pairs_mt(int mt, dim3 grid, hipStream_t s, const SgCall& c) {
+    switch (mt) {
+        case 1: sg_go<1, 3, SG_GLU | SG_RPAIR | EXTRA>(grid, s, c); break;
+        case 2: sg_go<2, 3, SG_GLU | SG_RPAIR | EXTRA>(grid, s, c); break;
+        default: sg_go<3, 3, SG_GLU | SG_RPAIR | EXTRA>(grid, s, c); break;
+    }
+}
+
 template <int EXTRA>
 void sg_dispatch(bool glu, int mt, int n_tiles, dim3 grid, hipStream_t s, const SgCall& c) {
     if constexpr (!(EXTRA & SG_RES)) {  // the residual form has no gate/up variant
@@ -802,6 +831,11 @@ extern "C" hipError_t ie_skinny_gemm_fused(const ie_bf16* x, int64_t x_stride, i
             sg_rows_mt<SG_SWZ | SG_LOOP>(mt, n_tiles, cus, stream, c);
     } else if (swz) {
         IE_SG_DISPATCH(SG_SWZ)
+    } else if (glu && sg_row_pairs(n / 2, n_tiles, mt)) {
+        c.nblk = 16 * n_tiles;
+        grid = dim3((unsigned)(n / 2 / 24));
+        if (norm) sg_row_pairs_mt<SG_NORM>(mt, grid, stream, c);
+        else sg_row_pairs_mt<SG_PLAIN>(mt, grid, stream, c);
     } else {
         IE_SG_DISPATCH(0)
     }
