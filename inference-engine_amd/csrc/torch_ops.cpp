@@ -539,6 +539,33 @@ void decode_attention_rope(const at::Tensor& q, const at::Tensor& k, const at::T
        "decode_attention_rope");
 }
 
+// The two with an output of their own, [B, Hq, D] like q (allocated here: from Python the
+// allocation costs as much host time as the launch).
+at::Tensor decode_attention_new(const at::Tensor& q, const at::Tensor& k_cache,
+                                const at::Tensor& v_cache, const at::Tensor& k_scale,
+                                const at::Tensor& v_scale, const at::Tensor& k_calibration,
+                                const at::Tensor& cached_lens, const at::Tensor& slot_ids,
+                                const at::Tensor& num_decoding, double scale,
+                                const c10::optional<at::Tensor>& plan) {
+    at::Tensor out = at::empty(q.sizes(), q.options());
+    decode_attention(q, k_cache, v_cache, k_scale, v_scale, k_calibration, cached_lens, slot_ids,
+                     num_decoding, scale, out, plan);
+    return out;
+}
+at::Tensor decode_attention_rope_new(
+    const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& q_norm_weight,
+    const at::Tensor& k_norm_weight, const at::Tensor& cos, const at::Tensor& sin,
+    const at::Tensor& k_cache, const at::Tensor& v_cache, const at::Tensor& k_scale,
+    const at::Tensor& v_scale, const at::Tensor& k_calibration, const at::Tensor& cached_lens,
+    const at::Tensor& slot_ids, const at::Tensor& num_decoding, double eps, double scale,
+    const c10::optional<at::Tensor>& plan) {
+    at::Tensor out = at::empty(q.sizes(), q.options());
+    decode_attention_rope(q, k, v, q_norm_weight, k_norm_weight, cos, sin, k_cache, v_cache,
+                          k_scale, v_scale, k_calibration, cached_lens, slot_ids, num_decoding,
+                          eps, scale, out, plan);
+    return out;
+}
+
 // The decode launch's work list for one step's metadata (ie_decode_attention_plan): int32
 // [grid, 4] on cached_lens' device, to pass to every layer's decode launch of that step.
 at::Tensor decode_plan(const at::Tensor& cached_lens, const at::Tensor& num_decoding,
@@ -772,6 +799,16 @@ TORCH_LIBRARY(ie, m) {
         "Tensor slot_ids, Tensor num_decoding, float eps, float scale, Tensor(e!) out, "
         "Tensor? plan=None) -> ()");
     m.def(
+        "decode_attention_new(Tensor q, Tensor k_cache, Tensor v_cache, Tensor k_scale, "
+        "Tensor v_scale, Tensor k_calibration, Tensor cached_lens, Tensor slot_ids, "
+        "Tensor num_decoding, float scale, Tensor? plan=None) -> Tensor");
+    m.def(
+        "decode_attention_rope_new(Tensor q, Tensor k, Tensor v, Tensor q_norm_weight, "
+        "Tensor k_norm_weight, Tensor cos, Tensor sin, Tensor(a!) k_cache, Tensor(b!) v_cache, "
+        "Tensor(c!) k_scale, Tensor(d!) v_scale, Tensor k_calibration, Tensor cached_lens, "
+        "Tensor slot_ids, Tensor num_decoding, float eps, float scale, Tensor? plan=None) "
+        "-> Tensor");
+    m.def(
         "decode_plan(Tensor cached_lens, Tensor num_decoding, int batch, int num_q_heads, "
         "int num_kv_heads) -> Tensor");
     m.def(
@@ -797,6 +834,13 @@ TORCH_LIBRARY(ie, m) {
     m.impl("decode_attention_workspace_size", &decode_attention_workspace_size);
 }
 
+// Not differentiable, and their outputs require no gradient whatever the inputs do, as an output
+// tensor passed in would not.
+TORCH_LIBRARY_IMPL(ie, Autograd, m) {
+    m.impl("decode_attention_new", torch::CppFunction::makeFallthrough());
+    m.impl("decode_attention_rope_new", torch::CppFunction::makeFallthrough());
+}
+
 TORCH_LIBRARY_IMPL(ie, CUDA, m) {
     m.impl("quantize_kv_prefill", &quantize_kv_prefill);
     m.impl("fused_rope_kv_decode", &fused_rope_kv_decode);
@@ -814,6 +858,8 @@ TORCH_LIBRARY_IMPL(ie, CUDA, m) {
     m.impl("skinny_weight_swizzle", &skinny_weight_swizzle);
     m.impl("decode_attention", &decode_attention);
     m.impl("decode_attention_rope", &decode_attention_rope);
+    m.impl("decode_attention_new", &decode_attention_new);
+    m.impl("decode_attention_rope_new", &decode_attention_rope_new);
     m.impl("dequantize_kv_prefix", &dequantize_kv_prefix);
     m.impl("prefill_attention", &prefill_attention);
     m.impl("prefill_plan", &prefill_plan);

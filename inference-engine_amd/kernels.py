@@ -67,7 +67,8 @@ def decode_attention(
     assert kv_cache.k_scale.stride() == kv_cache.v_scale.stride()
     B, Hq, D = q.shape
     if out is None:
-        out = torch.empty(B, Hq, D, device=q.device, dtype=q.dtype)
+        return ops().decode_attention_new(q, *_cache_args(kv_cache), cached_lens, slot_ids,
+                                          num_decoding, float(scale), plan)
     assert out.shape[0] >= B and out.shape[1:] == (Hq, D) and out.stride(-1) == 1
     ops().decode_attention(q, *_cache_args(kv_cache), cached_lens, slot_ids, num_decoding,
                            float(scale), out, plan)
@@ -122,7 +123,9 @@ def decode_attention_rope(
     assert kv_cache.k_scale.stride() == kv_cache.v_scale.stride()
     B, Hq, D = q.shape
     if out is None:
-        out = torch.empty(B, Hq, D, device=q.device, dtype=q.dtype)
+        return ops().decode_attention_rope_new(q, k, v, q_norm_weight, k_norm_weight, cos, sin,
+                                               *_cache_args(kv_cache), cached_lens, slot_ids,
+                                               num_decoding, float(eps), float(scale), plan)
     assert out.shape[0] >= B and out.shape[1:] == (Hq, D) and out.stride(-1) == 1
     ops().decode_attention_rope(q, k, v, q_norm_weight, k_norm_weight, cos, sin,
                                 *_cache_args(kv_cache), cached_lens, slot_ids, num_decoding,

@@ -97,3 +97,20 @@ def test_fused_form_many_heads_one_wave_workgroups(ie, dev):
     for name in ("k", "v", "k_scale", "v_scale"):
         assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)), name
     assert_attn_close(bf16_np(out), bf16_np(ref), "fused against two launches")
+
+
+def test_output_of_its_own(ie, workloads, dev):
+    """Without `out`: a contiguous [B, Hq, D] tensor whatever q's strides, that requires no gradient
+    whatever q does, with the values that a given `out` gets."""
+    wl = workloads.decode_workload([5, 300, 70], seed=76)
+    g = wl.to(dev)
+    wide = torch.randn(3, g.q.shape[1] + 4, 128, device=dev).bfloat16()
+    q = wide[:, 2:-2]
+    q.copy_(g.q)
+    args = (g.cache, g.cached_lens, g.slot_ids, g.num_decoding, SCALE)
+    out = torch.empty_like(g.q)
+    ie.decode_attention(g.q, *args, out=out)
+    own = ie.decode_attention(q.requires_grad_(), *args)
+    assert own.is_contiguous() and own.shape == g.q.shape and own.dtype == g.q.dtype
+    assert not own.requires_grad
+    assert torch.equal(own, out)
