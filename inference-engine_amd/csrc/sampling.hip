@@ -9,14 +9,15 @@
 //
 // sample_partial_kernel, grid (cdiv(V, block), B), 256 threads: the best (value, index) of each
 // block of a row's raw logits (sp_rounds), at tau != 0 with that entry's perturbed score.
-// sample_gumbel_kernel (tau != 0), the same grid: the best score of each block.
+// sample_gumbel_kernel (tau != 0), the same grid: the best score of each block. Small batches skip
+// the first launch at tau != 0: each block finds its own best raw entry (sample_launch).
 // sample_combine_kernel, grid B, one wave: the best over the row's blocks, and the seed increment
 // (after every block has read the seed: the launches are stream-ordered).
 //
 // Greedy is bound by HBM and launch latency (B x V logits read once). With noise, drawing a uniform
 // is what costs: Philox's 16 64-bit products take 16 cycles per wave each, 10 us for 32 x 151,936
 // entries on the whole chip. So entries that cannot win draw none: the noise is at most SP_GMAX, and
-// the best score of the row's block maxima bounds the winner's from below, so an entry whose
+// the best score of the row's block maxima (or of the block's own) bounds the winner's from below, so an entry whose
 // logit plus tau SP_GMAX stays under it is out. Float addition and multiplication are monotonic:
 // no winner is lost, whatever the logits. What is left is listed and drawn densely by the
 // workgroup, the hardware's fast logarithm first and the exact score only where that one plus its
@@ -116,11 +117,14 @@ __device__ __forceinline__ float noise_bound(float u) {
     return u > 0.9999f ? SP_GMAX : 0.05f - 0.69314718f * __builtin_amdgcn_logf(t);
 }
 
+// Eight entries at any element alignment (16-byte loads all the same: the device takes them
+// unaligned; rows of an odd vocabulary start anywhere).
 template <typename T>
 __device__ __forceinline__ void load8(const T* row, int64_t v, float (&x)[SP_VEC]);
 template <>
 __device__ __forceinline__ void load8<uint16_t>(const uint16_t* row, int64_t v, float (&x)[SP_VEC]) {
-    const uint4 w = *reinterpret_cast<const uint4*>(row + v);
+    uint4 w;
+    __builtin_memcpy(&w, row + v, sizeof(w));
     const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -130,22 +134,22 @@ __device__ __forceinline__ void load8<uint16_t>(const uint16_t* row, int64_t v, 
 }
 template <>
 __device__ __forceinline__ void load8<float>(const float* row, int64_t v, float (&x)[SP_VEC]) {
-    const float4 a = *reinterpret_cast<const float4*>(row + v);
-    const float4 b = *reinterpret_cast<const float4*>(row + v + 4);
+    float4 a, b;
+    __builtin_memcpy(&a, row + v, sizeof(a));
+    __builtin_memcpy(&b, row + v + 4, sizeof(b));
     x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
     x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
 
 // The workgroup's entries: thread tid holds 8 consecutive ones per round, [base + (r * 256 + tid) * 8,
-// +8); -inf past the row's end. `vec_ok`: V is a multiple of 8 and the row start 16-byte aligned, so
-// whole 8-entry groups load at once; otherwise entry by entry.
+// +8); -inf past the row's end.
 template <typename T, int ROUNDS>
-__device__ __forceinline__ void load_entries(const T* row, int64_t base, int64_t V, int vec_ok,
+__device__ __forceinline__ void load_entries(const T* row, int64_t base, int64_t V,
                                              float (&x)[ROUNDS][SP_VEC]) {
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
         const int64_t v0 = base + (int64_t)(r * SP_THREADS + threadIdx.x) * SP_VEC;
-        if (vec_ok && v0 + SP_VEC <= V) {
+        if (v0 + SP_VEC <= V) {
             load8<T>(row, v0, x[r]);
         } else {
 #pragma unroll
@@ -178,28 +182,35 @@ __device__ __forceinline__ Best block_best(Best best) {
     return best;
 }
 
+// The thread's best raw entry.
+template <int ROUNDS>
+__device__ __forceinline__ Best raw_best(const float (&x)[ROUNDS][SP_VEC], int64_t base,
+                                         int64_t V) {
+    Best best = {-INFINITY, 0x7fffffff};
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r)
+#pragma unroll
+        for (int j = 0; j < SP_VEC; ++j) {
+            const int64_t v = base + (int64_t)(r * SP_THREADS + threadIdx.x) * SP_VEC + j;
+            if (v < V) take(best, x[r][j], (int)v);
+        }
+    return best;
+}
+
 // grid (blocks, B), block 256: the best raw (value, index) of block bx of row by, to partial slot
 // by * gridDim.x + bx; at tau != 0 the value is that entry's perturbed score, the bound the next
 // launch starts from.
 template <typename T, int ROUNDS>
 __global__ __launch_bounds__(SP_THREADS) void sample_partial_kernel(
     const T* __restrict__ logits, int64_t ls, int64_t V, float tau,
-    const int64_t* __restrict__ seed, int vec_ok, float* __restrict__ pv, int* __restrict__ pi) {
+    const int64_t* __restrict__ seed, float* __restrict__ pv, int* __restrict__ pi) {
     const int b = blockIdx.y;
     const int64_t base = (int64_t)blockIdx.x * (SP_PASS * ROUNDS);
     const int tid = threadIdx.x;
     const uint64_t sd = (uint64_t)seed[0];
     float x[ROUNDS][SP_VEC];
-    load_entries<T, ROUNDS>(logits + b * ls, base, V, vec_ok, x);
-    Best best = {-INFINITY, 0x7fffffff};
-#pragma unroll
-    for (int r = 0; r < ROUNDS; ++r)
-#pragma unroll
-        for (int j = 0; j < SP_VEC; ++j) {
-            const int64_t v = base + (int64_t)(r * SP_THREADS + tid) * SP_VEC + j;
-            if (v < V) take(best, x[r][j], (int)v);
-        }
-    best = block_best(best);
+    load_entries<T, ROUNDS>(logits + b * ls, base, V, x);
+    Best best = block_best(raw_best<ROUNDS>(x, base, V));
     if (tid == 0) {
         if (tau != 0.f && best.i != 0x7fffffff)
             best.v = gumbel(best.v, tau,
@@ -210,12 +221,13 @@ __global__ __launch_bounds__(SP_THREADS) void sample_partial_kernel(
     }
 }
 
-// grid (blocks, B), block 256, after sample_partial_kernel at tau != 0: see the top. pv: that
-// launch's scores; bv, bi: this one's best (score, index) per block.
+// grid (blocks, B), block 256, at tau != 0: see the top. pv: sample_partial_kernel's scores, or null:
+// each block then bounds its entries by the score of its own largest one; bv, bi: the best (score,
+// index) per block.
 template <typename T, int ROUNDS>
 __global__ __launch_bounds__(SP_THREADS) void sample_gumbel_kernel(
     const T* __restrict__ logits, int64_t ls, int64_t V, float tau,
-    const int64_t* __restrict__ seed, int vec_ok, const float* __restrict__ pv,
+    const int64_t* __restrict__ seed, const float* __restrict__ pv,
     float* __restrict__ bv, int* __restrict__ bi) {
     const int b = blockIdx.y, nblk = gridDim.x;
     const T* row = logits + b * ls;
@@ -225,10 +237,22 @@ __global__ __launch_bounds__(SP_THREADS) void sample_gumbel_kernel(
     const uint32_t k0 = (uint32_t)sd, k1 = (uint32_t)(sd >> 32);
     const uint32_t row_off = (uint32_t)b * (uint32_t)V;
     float lb = -INFINITY;  // a score the row's best is at least
-    for (int j = lane; j < nblk; j += IE_WAVE) lb = fmaxf(lb, pv[b * nblk + j]);
+    if (pv)
+        for (int j = lane; j < nblk; j += IE_WAVE) lb = fmaxf(lb, pv[b * nblk + j]);
     float x[ROUNDS][SP_VEC];
-    load_entries<T, ROUNDS>(row, base, V, vec_ok, x);
-    lb = wave_max(lb);
+    load_entries<T, ROUNDS>(row, base, V, x);
+    if (pv) {
+        lb = wave_max(lb);
+    } else {  // small batches: the block's own bound
+        __shared__ float s_lb;
+        const Best top = block_best(raw_best<ROUNDS>(x, base, V));
+        if (tid == 0)
+            s_lb = top.i == 0x7fffffff
+                       ? -INFINITY
+                       : gumbel(top.v, tau, uniform_of(row_off + (uint32_t)top.i, k0, k1));
+        __syncthreads();
+        lb = s_lb;
+    }
     const float reach = fmaxf(tau * SP_GMAX, tau * SP_GMIN);
     uint32_t mask = 0;  // entries that may still win (those past the row's end may not)
 #pragma unroll
@@ -308,7 +332,8 @@ __global__ __launch_bounds__(64) void sample_combine_kernel(const float* __restr
 
 using namespace ie;
 
-// Per block of a row: the first launch's (value, index) and, at tau != 0, the second's.
+// Per block of a row: the first launch's (value, index) and, at tau != 0, the second's (whose place
+// does not depend on whether the first one ran).
 extern "C" size_t ie_sample_workspace_size(int32_t batch, int64_t vocab) {
     if (batch <= 0 || vocab <= 0) return 0;
     return (size_t)batch * (size_t)sp_blocks(batch, vocab) * 2 * (sizeof(float) + sizeof(int));
@@ -317,20 +342,25 @@ extern "C" size_t ie_sample_workspace_size(int32_t batch, int64_t vocab) {
 namespace {
 template <typename T, int ROUNDS>
 void sample_launch(const T* logits, int64_t ls, int32_t batch, int64_t vocab, float tau,
-                   int64_t* seed, int64_t* out, int64_t os, int vec_ok, void* workspace,
+                   int64_t* seed, int64_t* out, int64_t os, void* workspace,
                    int64_t nblk, hipStream_t stream) {
     const size_t n = (size_t)batch * (size_t)nblk;
     float* pv = reinterpret_cast<float*>(workspace);
     int* pi = reinterpret_cast<int*>(pv + n);
     const dim3 grid((unsigned)nblk, (unsigned)batch);
-    hipLaunchKernelGGL((sample_partial_kernel<T, ROUNDS>), grid, dim3(SP_THREADS), 0, stream,
-                       logits, ls, vocab, tau, (const int64_t*)seed, vec_ok, pv, pi);
+    // A row's bound is worth its launch from about five 2,048-entry workgroups per CU (151,936
+    // entries at tau 0.7, us in a graph / called back to back: 1 row 7.5 / 10.9 without it against
+    // 8.8 / 14.0, 16 rows 11.5 / 11.6 against 10.9 / 14.0, 24 rows 14.0 / 14.4 against 12.6 / 14.0).
+    const bool own = tau != 0.f && ROUNDS == 1 && batch * nblk <= 5 * device_cu_count();
+    if (!own)
+        hipLaunchKernelGGL((sample_partial_kernel<T, ROUNDS>), grid, dim3(SP_THREADS), 0, stream,
+                           logits, ls, vocab, tau, (const int64_t*)seed, pv, pi);
     if (tau != 0.f) {
         float* bv = reinterpret_cast<float*>(pi + n);
         int* bi = reinterpret_cast<int*>(bv + n);
         hipLaunchKernelGGL((sample_gumbel_kernel<T, ROUNDS>), grid, dim3(SP_THREADS), 0, stream,
-                           logits, ls, vocab, tau, (const int64_t*)seed, vec_ok, (const float*)pv,
-                           bv, bi);
+                           logits, ls, vocab, tau, (const int64_t*)seed,
+                           own ? (const float*)nullptr : (const float*)pv, bv, bi);
         pv = bv;
         pi = bi;
     }
@@ -340,14 +370,12 @@ void sample_launch(const T* logits, int64_t ls, int32_t batch, int64_t vocab, fl
 template <typename T>
 void sample_rounds(const void* logits, int64_t ls, int32_t batch, int64_t vocab, float tau,
                    int64_t* seed, int64_t* out, int64_t os, void* workspace, hipStream_t stream) {
-    const int vec_ok = vocab % SP_VEC == 0 && (ls * (int64_t)sizeof(T)) % 16 == 0 &&
-                       (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
     const int64_t nblk = sp_blocks(batch, vocab);
     if (sp_rounds(batch, vocab) == SP_ROUNDS)
-        sample_launch<T, SP_ROUNDS>((const T*)logits, ls, batch, vocab, tau, seed, out, os, vec_ok,
+        sample_launch<T, SP_ROUNDS>((const T*)logits, ls, batch, vocab, tau, seed, out, os,
                                     workspace, nblk, stream);
     else
-        sample_launch<T, 1>((const T*)logits, ls, batch, vocab, tau, seed, out, os, vec_ok,
+        sample_launch<T, 1>((const T*)logits, ls, batch, vocab, tau, seed, out, os,
                             workspace, nblk, stream);
 }
 }  // namespace

@@ -65,3 +65,14 @@ def test_candidates_around_the_list_capacity(ie, dev, extra):
         x[:, : block * 3 // 4 + extra] = 0.0
         x[:, 2 * block - 5:] = 0.0
         _check(ie, x, 1.0, 31 + extra, dev)
+
+
+@pytest.mark.parametrize("B", [1, 16, 17, 18, 24])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_batches_around_the_bound_launch(ie, dev, B, dtype):
+    """Up to five workgroups per CU a block bounds its entries by its own largest one (17 rows of 75
+    blocks are the last there on 256 CUs), above by the row's best; odd rows start unaligned."""
+    g = torch.Generator().manual_seed(B)
+    x = 2 * torch.randn(B, 151_937, generator=g)
+    x[:, torch.randint(0, 151_937, (30,), generator=g)] += 14 * torch.rand(30, generator=g)
+    _check(ie, x, 0.7, 40 + B, dev, dtype)
