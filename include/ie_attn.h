@@ -137,7 +137,8 @@ hipError_t ie_fused_rope_kv_decode(const ie_bf16* q, int64_t q_stride_b, int64_t
  * sequence and query head, the most any ratio uses, with room for max(batch, 1024) sequences of
  * max(num_q_heads, 128) heads, padded to 256 bytes), then fp32 split-K partials, head_dim + 2
  * values per (query head, work entry), where the work entries are at most the larger of
- * ie_decode_attention_grid(batch, units) for units = cdiv(num_q_heads, 2) and min(8, that). The arrival counts must be zero when a
+ * ie_decode_attention_grid(batch, units) for units = cdiv(num_q_heads, 2) and min(8, that). The
+ * arrival counts must be zero when a
  * workspace is first used (allocate it zeroed); every call that completes leaves them zero
  * again, so one workspace (of the largest size any of them needs) serves any number of calls in
  * stream order of any batch up to 1024 and any num_q_heads up to 128 (they share one count
@@ -242,8 +243,8 @@ hipError_t ie_decode_attention_noalloc(const ie_bf16* q, int64_t q_stride_b, int
  * The decode launch's work list, for tests and diagnostics: the work split of
  * qwen3-1.7b/kernels.py:20-70 (`compute_piece`, `assign_work`) as the decode kernel computes it
  * on the device. ie_decode_attention_grid(batch, num_units) is the number of work entries
- * (per unit: KV head x query-head pair, as above); ie_decode_attention_plan writes, for each entry
- * w, rows[4w .. 4w+3] = (sequence b, split index, splits of b, piece size in tokens), with
+ * (per unit: KV head x query-head pair, as above); ie_decode_attention_plan writes, for each
+ * entry w, rows[4w .. 4w+3] = (sequence b, split index, splits of b, piece size in tokens), with
  * splits = 0 for an entry that has no work. rows: int32 [grid, 4] device memory.
  */
 int32_t ie_decode_attention_grid(int32_t batch, int32_t num_units);

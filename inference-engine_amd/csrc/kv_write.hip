@@ -652,8 +652,9 @@ __global__ __launch_bounds__(256) void fused_norm_rope_prefill_kernel(
     }
 }
 
-// The same rows where they are 16-byte aligned (what an engine's packed rows are). What bounds it is HBM (each row read and written once); the kernel above moves two
-// bytes per lane and load, 128 bytes per instruction. Here a wave takes PP groups of four head rows
+// The same rows where they are 16-byte aligned (what an engine's packed rows are). What bounds it is
+// HBM (each row read and written once); the kernel above moves two bytes per lane and load, 128
+// bytes per instruction. Here a wave takes PP groups of four head rows
 // of one token: 16 lanes per row, lane c holding channels 8 c ... 8 c + 7 (one 16-byte load and
 // store), the second half of the row in lanes 8 ... 15, so the RoPE partner of a channel sits 8 lanes
 // away. Bit for bit the arithmetic above: the butterfly over 64 lanes becomes the same additions
@@ -910,9 +911,9 @@ extern "C" hipError_t ie_fused_norm_rope_prefill(
                             q_out_stride_head | k_out_stride_tok | k_out_stride_head;
     // (a few tokens of at most four rows finish sooner with a wave per row: 16 tokens of 2 + 1 heads
     // 2.3 against 2.4 us, 1,054 tokens 3.1 against 2.8)
-    if (!(rows <= 4 && num_tokens <= 512) && strides % 8 == 0 && aligned16(q) && aligned16(k) && aligned16(q_norm_weight) &&
-        aligned16(k_norm_weight) && aligned16(cos) && aligned16(sin) && aligned16(q_out) &&
-        aligned16(k_out)) {
+    if (!(rows <= 4 && num_tokens <= 512) && strides % 8 == 0 && aligned16(q) && aligned16(k) &&
+        aligned16(q_norm_weight) && aligned16(k_norm_weight) && aligned16(cos) && aligned16(sin) &&
+        aligned16(q_out) && aligned16(k_out)) {
         NormRopeArgs a{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)q_norm_weight,
                        (const uint16_t*)k_norm_weight, (const uint16_t*)cos, (const uint16_t*)sin,
                        q_stride_tok, q_stride_head, k_stride_tok, k_stride_head, cos_stride_tok,

@@ -17,8 +17,8 @@
 // Greedy is bound by HBM and launch latency (B x V logits read once). With noise, drawing a uniform
 // is what costs: Philox's 16 64-bit products take 16 cycles per wave each, 10 us for 32 x 151,936
 // entries on the whole chip. So entries that cannot win draw none: the noise is at most SP_GMAX, and
-// the best score of the row's block maxima (or of the block's own) bounds the winner's from below, so an entry whose
-// logit plus tau SP_GMAX stays under it is out. Float addition and multiplication are monotonic:
+// the best score of the row's block maxima (or of the block's own) bounds the winner's from below, so
+// an entry whose logit plus tau SP_GMAX stays under it is out. Float addition and multiplication are monotonic:
 // no winner is lost, whatever the logits. What is left is listed and drawn densely by the
 // workgroup, the hardware's fast logarithm first and the exact score only where that one plus its
 // error margin reaches the bound. 32 x 151,936 bf16, against every entry drawn with exact
