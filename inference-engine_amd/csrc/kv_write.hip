@@ -38,12 +38,9 @@ constexpr int QP_CAL_BLOCK = 256;  // chunk rows per workgroup of the separate c
 #ifndef IE_QS_WG_PER_CU
 #define IE_QS_WG_PER_CU 4
 #endif
-// The quantizers store int8 rows with the non-temporal cache policy: the cache is written once here
-// and read by later steps' attention, not by this launch (12,288-token step 22.8 -> 20.4 us; config
-// 4 level). Non-temporal loads of the bf16 rows measured slower. The scales do not take it: a wave
-// stores four rows' scales of K or V, 16 bytes, and a workgroup's such stores meet in a line of
-// the L2 before it goes to memory (non-temporal ones go one by one: 12,288 tokens in three chunks
-// 20.85 -> 20.25 us, 4,000 tokens of four KV heads 6.90 -> 6.49, 16,380 of eight level).
+// The quantizers store int8 rows and scales with the non-temporal cache policy: the cache is
+// written once here and read by later steps' attention, not by this launch (12,288-token step
+// 22.8 -> 20.4 us; config 4 level). Non-temporal loads of the bf16 rows measured slower.
 #ifndef IE_KV_NT_STORE
 #define IE_KV_NT_STORE 1
 #endif
@@ -57,6 +54,11 @@ __device__ __forceinline__ void row_store8(int8_t* p, uint2 v) {
     else
         *reinterpret_cast<uint2*>(p) = v;
 }
+__device__ __forceinline__ void scale_store(float* p, float v) {
+    if constexpr (IE_KV_NT_STORE) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // 8 consecutive bf16 (16 bytes), packed two per word.
 struct Row8 {
     uint32_t w[4];
@@ -169,7 +171,7 @@ __device__ __forceinline__ void quantize_store_kv_row(const uint32_t (&kw)[4],
         packed = pack_i8x8(qv);
     }
     row_store8(kc + col * stride_tok, packed);
-    if (c16 == 0) ks[col] = sk;
+    if (c16 == 0) scale_store(ks + col, sk);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         xv[2 * j] = bf16lo(vw[j]);
@@ -182,7 +184,7 @@ __device__ __forceinline__ void quantize_store_kv_row(const uint32_t (&kw)[4],
         packed = pack_i8x8(qv);
     }
     row_store8(vc + col * stride_tok, packed);
-    if (c16 == 0) vs[col] = sv;
+    if (c16 == 0) scale_store(vs + col, sv);
 }
 
 // The prefilling entries' chunks are cut into blocks of ROWS rows, numbered entry by entry.
