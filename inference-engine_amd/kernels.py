@@ -452,9 +452,10 @@ def tune_linear(weights: list, rows: list, calls: int = 20) -> None:
             use_skinny[(N, K, M)] = choice
             glu = {}
             if choice is not None and N % 64 == 0:
-                glu = {nt: _graph_time(cycle(lambda w, nt=nt: skinny_matmul_silu_mul(x, w, nt)))
+                glu = {nt: min(_graph_time(cycle(lambda w, nt=nt: skinny_matmul_silu_mul(x, w, nt)))
+                               for _ in range(2))
                        for nt in (1, 2) if (N // 2) % (16 * nt) == 0}
-                use_skinny_glu[(N, K, M)] = min(glu, key=glu.get)
+                use_skinny_glu[(N, K, M)] = _glu_width(glu)
             if choice is None:
                 continue
             mt = -(-M // 16)  # the reordered weight's width cannot be lowered to fit the LDS
@@ -477,6 +478,17 @@ def tune_linear(weights: list, rows: list, calls: int = 20) -> None:
             if glu:
                 use_skinny_glu_swz[(N, K, M)] = pick(swz_glu, min(glu.values()))
         del copies
+
+
+def _glu_width(times: dict) -> int:
+    """The tile width of the fused gate/up launch from its times: 2 unless 1 is over 3 % faster. The
+    two differ in the order of the partial sums, i.e. in result bits, and at many column counts both
+    run the same 24-column workgroups (12.5 and 12.4 us at [12288, 2048], 32 rows): the faster of two
+    equal times would choose the bits by noise, anew in every process. Where the launches differ,
+    width 1 wins by 3 to 40 % (short weights, 24,576 columns at few rows) or not at all."""
+    if 1 in times and 2 in times:
+        return 1 if times[1] < 0.97 * times[2] else 2
+    return min(times, key=times.get)
 
 
 def _graph_time(fns: list) -> float:
