@@ -185,7 +185,8 @@ int32_t ie_decode_attention_target(int32_t batch, int32_t num_units);
  *   out[b, h] = sum_t softmax_t(scale * k_scale[t] * <q[b, h], k[t]>) * v_scale[t] * v[t].
  * Only rows b < num_decoding[0] of out are written. `workspace` must hold
  * ie_decode_attention_workspace_size(B, num_q_heads, head_dim) bytes with its arrival counts
- * zero (see there); calls that share a workspace must not overlap.
+ * zero (see there); calls that share a workspace must not overlap. batch: under 4 million (the work
+ * entries per head number less than 2^22).
  */
 hipError_t ie_decode_attention(const ie_bf16* q, int64_t q_stride_b, int64_t q_stride_h,
                                int32_t batch, int32_t num_q_heads, const ie_kv_cache* cache,

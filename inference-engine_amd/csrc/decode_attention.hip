@@ -61,6 +61,7 @@ constexpr int DA_WAVES_PER_CU = 8;
 constexpr int DA_MIN_PIECE = 128;
 constexpr int DA_MAX_SPLITS = 1024;  // per-KV-head workgroup target, at most
 constexpr int DA_D = 128;
+constexpr int DA_MAX_WORK = 1 << 22;  // work entries per head, at most (the merge's 32-bit offsets)
 constexpr uint32_t K64 = 0x64646464u;
 
 // Workgroup target per unit (a KV head in a launch; see decode_units for work lists) of workgroups
@@ -614,10 +615,18 @@ decode_attention_kernel(DecodeArgs a) {
     // device-coherent stores and counts itself in; the last to arrive merges them all
     // (kernels.py:216-264, in base 2, pieces in order) and resets the count for the next call.
     if (!arrive_last(a.arrivals + b * a.hkv + hk, needed)) return;
-    const rsrc_t pr = make_rsrc(a.part_acc, (uint32_t)((int64_t)a.hq * a.nwork * DA_D * 4));
     for (int q = tid; q < quads; q += THREADS) {
         const int h = q >> 5, d = 4 * (q & 31);
         const int64_t row0 = (int64_t)(qh0 + h) * a.nwork + (item - split);
+        // The wave's two heads from the sequence's first partial of the first one: 32-bit offsets
+        // reach them whatever the head count and the batch (nwork < DA_MAX_WORK), where offsets into
+        // all partials passed 4 GiB at 128 heads of 65,536 sequences. (8-byte loads from 64-bit
+        // addresses instead: 64 pieces of 64/4 heads 26.1 us against 21.6.)
+        const int h0 = uniform(h);
+        const rsrc_t pr =
+            make_rsrc(a.part_acc + ((int64_t)(qh0 + h0) * a.nwork + (item - split)) * DA_D,
+                      (uint32_t)(a.nwork + needed) * (DA_D * 4));
+        const uint32_t off0 = (uint32_t)((h - h0) * a.nwork * DA_D + d) * 4;
         constexpr int CB = 8;  // partials in flight: one round trip each batch
         f32x4_t av[CB];
         float pm[CB], pl[CB];
@@ -627,7 +636,7 @@ decode_attention_kernel(DecodeArgs a) {
                 const bool in = s0 + v < needed;
                 av[v] = __builtin_bit_cast(
                     f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                 pr, in ? (int)(((row0 + s0 + v) * DA_D + d) * 4) : -64, 0, CPOL_SC1));
+                                 pr, in ? (int)(off0 + (s0 + v) * (DA_D * 4)) : -64, 0, CPOL_SC1));
                 pm[v] = in ? ld_dev(a.part_m + row0 + s0 + v) : -INFINITY;
                 pl[v] = in ? ld_dev(a.part_l + row0 + s0 + v) : 0.0f;
             }
@@ -834,6 +843,7 @@ static hipError_t check_decode(const ie_bf16* q, int32_t batch, int32_t num_q_he
                    ((reinterpret_cast<uintptr_t>(q) & 15) == 0 && q_sb % 8 == 0 && q_sh % 8 == 0),
                "q rows must be 16-byte aligned with contiguous head_dim");
     *L = call_layout(batch, num_q_heads, (int)cache->num_kv_heads, max_bytes);
+    IE_REQUIRE(L->nwork < DA_MAX_WORK, "batch too large");
     IE_REQUIRE(workspace != nullptr && workspace_bytes >= L->bytes, "workspace too small");
     IE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "workspace must be aligned");
     return hipSuccess;
