@@ -436,7 +436,8 @@ hipError_t ie_prefill_attention_planned(
  * key (low, high 32 bits of *seed), first output word x as int32,
  * u = float(x < 0 ? -x - 1 : x) * 4.6566127342e-10. At tau = 0 no uniform is drawn. *seed (a
  * device int64) is incremented once per call, after every row has read it, also when batch is
- * 0. `workspace` must hold ie_sample_workspace_size(batch, vocab) bytes.
+ * 0. `workspace` must hold ie_sample_workspace_size(batch, vocab) bytes (a size that never falls as
+ * either grows).
  */
 size_t ie_sample_workspace_size(int32_t batch, int64_t vocab);
 hipError_t ie_sample(const void* logits, int32_t logits_dtype, int64_t logits_stride_row,
