@@ -33,6 +33,7 @@ constexpr int SP_THREADS = 256;
 constexpr int SP_VEC = 8;                                // entries per 16-byte bf16 load
 constexpr int SP_PASS = SP_THREADS * SP_VEC;             // 2048 entries per load of a workgroup
 constexpr int SP_ROUNDS = 2;                             // loads per thread, or 1
+constexpr int64_t SP_MAX_VOCAB = 65535LL * 8192;         // at most (indices fit int32)
 // No uniform's noise exceeds 15.95 (u <= 0.99999988) or falls below -3.14 (u >= 1e-10).
 constexpr float SP_GMAX = 16.0f, SP_GMIN = -4.0f;
 // Loads per thread for a batch of rows: blocks of 4096 entries while they give each CU four
@@ -216,8 +217,9 @@ __global__ __launch_bounds__(SP_THREADS) void sample_partial_kernel(
             best.v = gumbel(best.v, tau,
                             uniform_of((uint32_t)b * (uint32_t)V + (uint32_t)best.i, (uint32_t)sd,
                                        (uint32_t)(sd >> 32)));
-        pv[b * gridDim.x + blockIdx.x] = best.v;
-        pi[b * gridDim.x + blockIdx.x] = best.i;
+        const int64_t slot = (int64_t)b * gridDim.x + blockIdx.x;
+        pv[slot] = best.v;
+        pi[slot] = best.i;
     }
 }
 
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(SP_THREADS) void sample_gumbel_kernel(
     const uint32_t row_off = (uint32_t)b * (uint32_t)V;
     float lb = -INFINITY;  // a score the row's best is at least
     if (pv)
-        for (int j = lane; j < nblk; j += IE_WAVE) lb = fmaxf(lb, pv[b * nblk + j]);
+        for (int j = lane; j < nblk; j += IE_WAVE) lb = fmaxf(lb, pv[(int64_t)b * nblk + j]);
     float x[ROUNDS][SP_VEC];
     load_entries<T, ROUNDS>(row, base, V, x);
     if (pv) {
@@ -307,8 +309,9 @@ __global__ __launch_bounds__(SP_THREADS) void sample_gumbel_kernel(
     }
     best = block_best(best);
     if (tid == 0) {
-        bv[b * nblk + blockIdx.x] = best.v;
-        bi[b * nblk + blockIdx.x] = best.i;
+        const int64_t slot = (int64_t)b * nblk + blockIdx.x;
+        bv[slot] = best.v;
+        bi[slot] = best.i;
     }
 }
 
@@ -321,7 +324,8 @@ __global__ __launch_bounds__(64) void sample_combine_kernel(const float* __restr
     const int b = blockIdx.x, lane = threadIdx.x;
     if (b < B) {
         Best best = {-INFINITY, 0x7fffffff};
-        for (int j = lane; j < nblk; j += IE_WAVE) take(best, pv[b * nblk + j], pi[b * nblk + j]);
+        const int64_t row = (int64_t)b * nblk;
+        for (int j = lane; j < nblk; j += IE_WAVE) take(best, pv[row + j], pi[row + j]);
         best = wave_best(best);
         if (lane == 0) out[b * os] = best.i;
     }
@@ -401,8 +405,7 @@ extern "C" hipError_t ie_sample(const void* logits, int32_t logits_dtype, int64_
     }
     IE_REQUIRE(logits && out && workspace, "null pointer");
     IE_REQUIRE(workspace_bytes >= ie_sample_workspace_size(batch, vocab), "workspace too small");
-    IE_REQUIRE((vocab + SP_PASS * SP_ROUNDS - 1) / (SP_PASS * SP_ROUNDS) < 65536,
-               "vocab too large");
+    IE_REQUIRE(vocab <= SP_MAX_VOCAB, "vocab too large");
     if (logits_dtype == IE_DTYPE_BF16)
         sample_rounds<uint16_t>(logits, logits_stride_row, batch, vocab, tau, seed, out,
                                 out_stride_row, workspace, stream);

@@ -76,3 +76,15 @@ def test_batches_around_the_bound_launch(ie, dev, B, dtype):
     x = 2 * torch.randn(B, 151_937, generator=g)
     x[:, torch.randint(0, 151_937, (30,), generator=g)] += 14 * torch.rand(30, generator=g)
     _check(ie, x, 0.7, 40 + B, dev, dtype)
+
+
+@pytest.mark.parametrize("V", [2 ** 28, 2 ** 28 + 4099])
+@pytest.mark.parametrize("tau", [0.0, 0.7])
+def test_vocabularies_past_2_28(ie, dev, V, tau):
+    """Entries that no noise can lift past the one planted far above them, in the last block."""
+    say(f"sample 1 x {V} tau={tau}")
+    x = torch.full((1, V), -20.0, dtype=torch.bfloat16, device=dev)
+    x[0, V - 3] = 30.0
+    seed = torch.tensor([9], dtype=torch.int64, device=dev)
+    assert int(ie.sample(x, tau, seed).item()) == V - 3
+    assert int(seed.item()) == 10
