@@ -793,7 +793,12 @@ static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes) {
     auto entries = [&](int t) { return batch <= t ? t : t + batch; };
     int waves = decode_waves(batch, hkv), target = decode_target(hkv, waves);
     while (entries(target) > fit && waves < 8) target = decode_target(hkv, waves *= 2);
-    if (entries(target) > fit) target = std::max(1, batch <= fit ? fit : fit - batch);
+    if (entries(target) > fit) {
+        // in the widest workgroups of which every entry is resident (one-wave ones where none is):
+        // 12/4 heads B=300 have 341 entries a head, 5 rounds of 8-wave workgroups
+        target = std::max(1, batch <= fit ? fit : fit - batch);
+        while (waves > 1 && decode_target(hkv, waves) < entries(target)) waves /= 2;
+    }
     return layout_of(batch, hq, waves, target);
 }
 
