@@ -137,22 +137,21 @@ hipError_t ie_fused_rope_kv_decode(const ie_bf16* q, int64_t q_stride_b, int64_t
  * sequence and query head, the most any ratio uses, with room for max(batch, 1024) sequences of
  * max(num_q_heads, 128) heads, padded to 256 bytes), then fp32 split-K partials, head_dim + 2
  * values per (query head, work entry), where the work entries are at most the larger of
- * ie_decode_attention_grid(batch, units) for units = cdiv(num_q_heads, 2) and min(8, that). The
- * arrival counts must be zero when a
- * workspace is first used (allocate it zeroed); every call that completes leaves them zero
- * again, so one workspace (of the largest size any of them needs) serves any number of calls in
- * stream order of any batch up to 1024 and any num_q_heads up to 128 (they share one count
- * region). A workspace used with a larger batch or head count serves that shape only, unless
- * zeroed again.
+ * ie_decode_attention_grid(batch, units) for units = cdiv(num_q_heads, 2) and min(8, that) (a launch
+ * whose KV heads would give it more entries has as many as fit). The arrival counts must be zero when
+ * a workspace is first used (allocate it zeroed); every call that completes leaves them zero again,
+ * so one workspace (of the largest size any of them needs) serves any number of calls in stream order
+ * of any batch up to 1024 and any num_q_heads up to 128 (they share one count region). A workspace
+ * used with a larger batch or head count serves that shape only, unless zeroed again.
  */
 size_t ie_decode_attention_workspace_size(int32_t batch, int32_t num_q_heads, int32_t head_dim);
 
 /*
  * The leading bytes of a decode workspace for `batch` sequences that must be zero on entry (the
- * arrival counts: max(batch, 1024) * num_kv_heads uint32, padded to 256 bytes). Zeroing them
- * resets a workspace, e.g. one whose memory was reused or a launch that did not complete, and
+ * arrival counts: max(batch, 1024) * max(num_q_heads, 128) uint32, padded to 256 bytes). Zeroing
+ * them resets a workspace, e.g. one whose memory was reused or a launch that did not complete, and
  * a caller that records the decode call into a hipGraph from freshly allocated memory records
- * a fill of these bytes first. (max(batch, 1024) * num_q_heads uint32, padded to 256 bytes.) No counterpart in the reference (its partials need no counts).
+ * a fill of these bytes first. No counterpart in the reference (its partials need no counts).
  */
 size_t ie_decode_attention_workspace_counts_bytes(int32_t batch, int32_t num_q_heads);
 
@@ -209,7 +208,7 @@ hipError_t ie_decode_attention(const ie_bf16* q, int64_t q_stride_b, int64_t q_s
  * slot_ids[b]), and out[b] is decode attention with the q that ie_fused_rope_kv_decode would
  * return (its bits); q_out itself is not produced. Within the launch the piece of each sequence
  * that ends at the new token computes that token's K/V row, writes it to the cache and uses its
- * own copy (in LDS); no piece reads that column from the cache.
+ * own copy (in LDS); no piece uses what the cache held in that column.
  */
 hipError_t ie_decode_attention_rope(
     const ie_bf16* q, int64_t q_stride_b, int64_t q_stride_h, const ie_bf16* k,
@@ -275,8 +274,8 @@ hipError_t ie_decode_step_prologue(const int32_t* cached_lens, const int32_t* nu
  * ie_decode_attention_plan wrote for the same cached_lens and num_decoding values, batch,
  * num_units (KV heads x query-head pairs) and device, 16-byte aligned, and plan_rows, their
  * count (at least ie_decode_attention_grid(batch, num_units)). Each workgroup reads its entry in
- * one load instead of deriving the work split from cached_lens (GQA ratios 1 and 2; launches above
- * cut other entries and derive them from cached_lens all the same). For engines that run every
+ * one load instead of deriving the work split from cached_lens (where the launch's entries are the
+ * list's, as at GQA ratio 2; else it derives them from cached_lens all the same). For engines that run every
  * layer of a decode step over one step's metadata: compute the plan once per step. A plan that
  * does not match the arguments is undefined behaviour (its rows name the sequences, pieces and
  * merges of each workgroup).

@@ -784,20 +784,29 @@ static Layout workspace_size_layout(int batch, int hq) {
 // the same rule per KV head, but the partials of all heads of an entry must fit the workspace of
 // workspace_size_layout (and max_bytes, what the call may count on at most): where they do not,
 // workgroups of twice the waves and half the entries, up to 8 waves (one per CU), then as many
-// entries as fit (few KV heads only: at 8 the first rule always fits).
-static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes) {
-    if (hq <= 2 * hkv) return workspace_layout(batch, hq, hkv);
-    const Layout S = workspace_size_layout(batch, hq);
+// entries as fit (few KV heads only: at 8 the first rule always fits). At ratio 1 a batch can pass
+// the largest target of Hkv units, which adds spare entries, while the workspace's fewer units still
+// hold it without (16/16 heads B=129-256 on 256 CUs: 257-384 entries, 256 reserved): the entries
+// reserved, then.
+static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes = SIZE_MAX) {
+    const Layout S = workspace_size_layout(batch, hq), own = workspace_layout(batch, hq, hkv);
+    // the widest workgroups of which every entry is resident (one-wave ones where none is): 12/4
+    // heads B=300 have 341 entries a head, 5 rounds of 8-wave workgroups
+    auto resident_waves = [&](int entries) {
+        int w = 8;
+        while (w > 1 && decode_target(hkv, w) < entries) w /= 2;
+        return w;
+    };
+    if (hq <= 2 * hkv)
+        return own.bytes <= S.bytes ? own : layout_of(batch, hq, resident_waves(S.nwork), S.target);
     const size_t room = std::min(S.bytes, max_bytes), row = (DA_D + 2) * sizeof(float);
     const int fit = room > S.acc_off ? (int)((room - S.acc_off) / (hq * row)) : 0;
     auto entries = [&](int t) { return batch <= t ? t : t + batch; };
-    int waves = decode_waves(batch, hkv), target = decode_target(hkv, waves);
+    int waves = own.waves, target = own.target;
     while (entries(target) > fit && waves < 8) target = decode_target(hkv, waves *= 2);
     if (entries(target) > fit) {
-        // in the widest workgroups of which every entry is resident (one-wave ones where none is):
-        // 12/4 heads B=300 have 341 entries a head, 5 rounds of 8-wave workgroups
         target = std::max(1, batch <= fit ? fit : fit - batch);
-        while (waves > 1 && decode_target(hkv, waves) < entries(target)) waves /= 2;
+        waves = resident_waves(entries(target));
     }
     return layout_of(batch, hq, waves, target);
 }
@@ -894,7 +903,9 @@ static hipError_t decode_launch(DecodeArgs& a, const Layout& L, hipStream_t stre
     // resident slots while they find out that they are idle
     const dim3 grid((unsigned)L.nwork, (unsigned)a.hkv);
     a.out_vec = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && a.o_sb % 4 == 0 && a.o_sh % 4 == 0;
-    if (a.ratio > 2) a.plan = nullptr;  // a list of other entries (decode_units)
+    // a list is read where it has the launch's entries: they depend on the batch and the target alone
+    if (a.plan && ie_decode_attention_target(a.batch, decode_units(a.hq, a.hkv)) != a.target)
+        a.plan = nullptr;
     switch (L.waves) {
         case 8: hipLaunchKernelGGL((decode_attention_kernel<8, ROPE>), grid, dim3(512), 0, stream, a); break;
         case 4: hipLaunchKernelGGL((decode_attention_kernel<4, ROPE>), grid, dim3(256), 0, stream, a); break;

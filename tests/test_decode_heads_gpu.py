@@ -45,6 +45,22 @@ def test_narrow_workgroups(ie, workloads, dev, batch, hq, hkv):
     assert_attn_close(_run(ie, wl, dev), _ref(wl), f"B={batch} {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("batch,heads", [(129, 16), (256, 16), (257, 16), (257, 8), (100, 7), (65, 32)])
+def test_batches_past_a_target_at_ratio_1(ie, workloads, dev, batch, heads):
+    """Batches that pass the largest target of as many units as KV heads: the entries are cut to the
+    workspace, which is sized by the query heads alone."""
+    say(f"decode B={batch} {heads}/{heads}")
+    ctx = [EDGES[i % 15] for i in range(batch)]
+    wl = workloads.decode_workload(ctx, seed=77, hq=heads, hkv=heads)
+    out = _run(ie, wl, dev)
+    assert_attn_close(out, _ref(wl), f"B={batch} {heads}/{heads}")
+    g = wl.to(dev)
+    planned = ie.decode_attention(g.q, g.cache, g.cached_lens, g.slot_ids, g.num_decoding, SCALE,
+                                  plan=ie.decode_plan(g.cached_lens, g.num_decoding, batch, heads,
+                                                      heads))
+    assert np.array_equal(bf16_np(planned), out)
+
+
 def test_out_rows_without_8_byte_alignment(ie, workloads, dev):
     wl = workloads.decode_workload([33, 2000, 700], seed=73, hq=32, hkv=8)
     buf = torch.full((3, 32, 131), 5.0, dtype=torch.bfloat16, device=dev)
