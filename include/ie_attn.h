@@ -155,16 +155,24 @@ size_t ie_decode_attention_workspace_size(int32_t batch, int32_t num_q_heads, in
  */
 size_t ie_decode_attention_workspace_counts_bytes(int32_t batch, int32_t num_q_heads);
 
+/*
+ * num_units for the work list of a launch of num_q_heads over num_kv_heads heads and `batch`
+ * sequences on the current device: mostly num_kv_heads (one unit per KV head), more where the
+ * entries of so few units would not fit ie_decode_attention_workspace_size. A list made for them is
+ * read at every GQA ratio (plan_rows of ie_decode_attention_planned); a few batches above ratio 2
+ * have entries that no list has, and derive them. 0 for head counts that are no multiple. No
+ * counterpart in the reference.
+ */
+int32_t ie_decode_attention_units(int32_t batch, int32_t num_q_heads, int32_t num_kv_heads);
+
 /* The largest per-unit workgroup target of any launch shape (CUs * 8 / num_units, one-wave
- * workgroups): an upper bound on splits per sequence at GQA ratios 1 and 2. A unit of a work list
- * is a KV head and one pair of its query heads: num_units = num_kv_heads *
- * cdiv(num_q_heads / num_kv_heads, 2), num_kv_heads itself at ratios 1 and 2. Launches above
- * ratio 2 cut their entries per KV head and read no list (see ie_decode_attention_planned). */
+ * workgroups): an upper bound on the splits of a sequence in a launch cut for num_units (num_kv_heads:
+ * in any launch over that many KV heads). */
 int32_t ie_decode_attention_max_splits(int32_t num_units);
 
 /*
  * The per-unit workgroup target of the work split (qwen3-1.7b/kernels.py:20-37 TARGET) that
- * a work list uses for `batch` sequences on the current device (num_units as above). A launch
+ * a work list uses for `batch` sequences on the current device. A launch
  * fills the CUs with 8 waves each, as 4-wave workgroups (target CUs * 2 / num_units)
  * while the batch fits that target, else as 2-wave (CUs * 4 / num_units) or one-wave (CUs * 8 /
  * num_units) workgroups, the first whose target holds the batch (the one-wave one above that).
@@ -242,9 +250,9 @@ hipError_t ie_decode_attention_noalloc(const ie_bf16* q, int64_t q_stride_b, int
 /*
  * The decode launch's work list, for tests and diagnostics: the work split of
  * qwen3-1.7b/kernels.py:20-70 (`compute_piece`, `assign_work`) as the decode kernel computes it
- * on the device. ie_decode_attention_grid(batch, num_units) is the number of work entries
- * (per unit: KV head x query-head pair, as above); ie_decode_attention_plan writes, for each
- * entry w, rows[4w .. 4w+3] = (sequence b, split index, splits of b, piece size in tokens), with
+ * on the device. ie_decode_attention_grid(batch, num_units) is the number of work entries (num_units:
+ * ie_decode_attention_units, or KV heads x query-head pairs, num_kv_heads * cdiv(num_q_heads /
+ * num_kv_heads, 2)); ie_decode_attention_plan writes, for each entry w, rows[4w .. 4w+3] = (sequence b, split index, splits of b, piece size in tokens), with
  * splits = 0 for an entry that has no work. rows: int32 [grid, 4] device memory.
  */
 int32_t ie_decode_attention_grid(int32_t batch, int32_t num_units);
@@ -272,14 +280,17 @@ hipError_t ie_decode_step_prologue(const int32_t* cached_lens, const int32_t* nu
  * ie_decode_attention and ie_decode_attention_rope with their work list precomputed (no
  * counterpart in the reference): the same arguments and results, plus `plan`, the rows
  * ie_decode_attention_plan wrote for the same cached_lens and num_decoding values, batch,
- * num_units (KV heads x query-head pairs) and device, 16-byte aligned, and plan_rows, their
- * count (at least ie_decode_attention_grid(batch, num_units)). Each workgroup reads its entry in
- * one load instead of deriving the work split from cached_lens (where the launch's entries are the
- * list's, as at GQA ratio 2; else it derives them from cached_lens all the same). For engines that run every
+ * num_units and device, 16-byte aligned, and plan_rows, their count (at least
+ * ie_decode_attention_grid(batch, num_units)), plus IE_PLAN_LAUNCH_UNITS where num_units is
+ * ie_decode_attention_units(batch, num_q_heads, num_kv_heads); without it num_units is KV heads x
+ * query-head pairs. Each workgroup reads its entry in one load instead of deriving the work split
+ * from cached_lens (where the launch's entries are the list's: the two unit counts are the same at
+ * GQA ratios 1 and 2; else it derives them all the same). For engines that run every
  * layer of a decode step over one step's metadata: compute the plan once per step. A plan that
  * does not match the arguments is undefined behaviour (its rows name the sequences, pieces and
  * merges of each workgroup).
  */
+#define IE_PLAN_LAUNCH_UNITS ((int64_t)1 << 62)
 hipError_t ie_decode_attention_planned(
     const ie_bf16* q, int64_t q_stride_b, int64_t q_stride_h, int32_t batch, int32_t num_q_heads,
     const ie_kv_cache* cache, const int32_t* cached_lens, const int32_t* slot_ids,

@@ -77,9 +77,8 @@ int decode_waves(int batch, int units) {
         if (batch <= decode_target(units, w)) return w;
     return 1;
 }
-// Units a work list is made for: KV heads x query-head pairs per KV head, the KV heads at ratios
-// 1 and 2. Launches of those ratios run from such a list; above ratio 2 a launch cuts its entries
-// per KV head (call_layout) and derives them itself.
+// Units a work list is taken to be made for: KV heads x query-head pairs per KV head, the KV heads at
+// ratios 1 and 2; with IE_PLAN_LAUNCH_UNITS, what the launch is cut for (list_units).
 int decode_units(int hq, int hkv) { return hkv * ((hq / std::max(1, hkv) + 1) / 2); }
 
 
@@ -811,6 +810,15 @@ static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes = SIZE_MA
     return layout_of(batch, hq, waves, target);
 }
 
+// The num_units whose work list has a call's entries (a list depends on the batch and the target
+// alone), or 0: none of the unit counts that a layout comes from gives that target.
+static int list_units(int batch, int hq, int hkv) {
+    const int target = call_layout(batch, hq, hkv).target, pairs = std::max(1, (hq + 1) / 2);
+    for (int u : {hkv, 2 * hkv, 4 * hkv, 8 * hkv, std::min(8, pairs), pairs})
+        if (workspace_layout(batch, hq, u).target == target) return u;
+    return 0;
+}
+
 }  // namespace ie
 
 using namespace ie;
@@ -828,6 +836,13 @@ extern "C" int32_t ie_decode_attention_max_splits(int32_t num_units) {
 extern "C" int32_t ie_decode_attention_target(int32_t batch, int32_t num_units) {
     if (batch <= 0 || num_units <= 0) return 0;
     return decode_target(num_units, decode_waves(batch, num_units));
+}
+
+extern "C" int32_t ie_decode_attention_units(int32_t batch, int32_t num_q_heads,
+                                             int32_t num_kv_heads) {
+    if (num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads) return 0;
+    const int units = list_units(std::max(batch, 0), num_q_heads, num_kv_heads);
+    return units ? units : decode_units(num_q_heads, num_kv_heads);
 }
 
 extern "C" size_t ie_decode_attention_workspace_size(int32_t batch, int32_t num_q_heads,
@@ -903,9 +918,6 @@ static hipError_t decode_launch(DecodeArgs& a, const Layout& L, hipStream_t stre
     // resident slots while they find out that they are idle
     const dim3 grid((unsigned)L.nwork, (unsigned)a.hkv);
     a.out_vec = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && a.o_sb % 4 == 0 && a.o_sh % 4 == 0;
-    // a list is read where it has the launch's entries: they depend on the batch and the target alone
-    if (a.plan && ie_decode_attention_target(a.batch, decode_units(a.hq, a.hkv)) != a.target)
-        a.plan = nullptr;
     switch (L.waves) {
         case 8: hipLaunchKernelGGL((decode_attention_kernel<8, ROPE>), grid, dim3(512), 0, stream, a); break;
         case 4: hipLaunchKernelGGL((decode_attention_kernel<4, ROPE>), grid, dim3(256), 0, stream, a); break;
@@ -915,13 +927,18 @@ static hipError_t decode_launch(DecodeArgs& a, const Layout& L, hipStream_t stre
     return hipGetLastError();
 }
 
-// A precomputed work list must cover the grid it is made for.
+// A precomputed work list must cover the grid it is made for; it is read (*read) where that is the
+// launch's.
 static hipError_t check_plan(const int32_t* plan, int64_t plan_rows, int32_t batch, int32_t hq,
-                             int32_t hkv) {
+                             int32_t hkv, const Layout& L, bool* read) {
     IE_REQUIRE(plan != nullptr, "null plan");
-    IE_REQUIRE(plan_rows >= ie_decode_attention_grid(batch, decode_units(hq, hkv)),
+    const bool launch = plan_rows >= IE_PLAN_LAUNCH_UNITS;
+    const int units = launch ? ie_decode_attention_units(batch, hq, hkv) : decode_units(hq, hkv);
+    if (launch) plan_rows -= IE_PLAN_LAUNCH_UNITS;
+    IE_REQUIRE(plan_rows >= ie_decode_attention_grid(batch, units),
                "plan must hold ie_decode_attention_grid(batch, units) rows");
     IE_REQUIRE((reinterpret_cast<uintptr_t>(plan) & 15) == 0, "plan must be 16-byte aligned");
+    *read = ie_decode_attention_target(batch, units) == L.target;
     return hipSuccess;
 }
 
@@ -937,13 +954,14 @@ static hipError_t decode_plain(const ie_bf16* q, int64_t q_stride_b, int64_t q_s
                                 out, q_stride_b, q_stride_h, workspace, workspace_bytes, &L, true,
                                 max_bytes);
     if (e != hipSuccess || batch == 0) return e;
+    bool read = false;
     if (planned && (e = check_plan(plan, plan_rows, batch, num_q_heads,
-                                   (int32_t)cache->num_kv_heads)) != hipSuccess)
+                                   (int32_t)cache->num_kv_heads, L, &read)) != hipSuccess)
         return e;
     DecodeArgs a = decode_args(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens,
                                slot_ids, num_decoding, scale, out, out_stride_b, out_stride_h,
                                workspace, L);
-    a.plan = planned ? plan : nullptr;
+    a.plan = read ? plan : nullptr;
     return decode_launch<false>(a, L, stream);
 }
 
@@ -984,13 +1002,14 @@ static hipError_t decode_rope(
                                 false);
     if (e != hipSuccess || batch == 0) return e;
     IE_REQUIRE(k && v && q_norm_weight && k_norm_weight && cos && sin, "null pointer");
+    bool read = false;
     if (planned && (e = check_plan(plan, plan_rows, batch, num_q_heads,
-                                   (int32_t)cache->num_kv_heads)) != hipSuccess)
+                                   (int32_t)cache->num_kv_heads, L, &read)) != hipSuccess)
         return e;
     DecodeArgs a = decode_args(q, q_stride_b, q_stride_h, batch, num_q_heads, cache, cached_lens,
                                slot_ids, num_decoding, scale, out, out_stride_b, out_stride_h,
                                workspace, L);
-    a.plan = planned ? plan : nullptr;
+    a.plan = read ? plan : nullptr;
     a.k_new = (const uint16_t*)k;
     a.k_sb = k_stride_b;
     a.k_sh = k_stride_h;

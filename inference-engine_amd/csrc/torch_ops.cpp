@@ -375,6 +375,13 @@ void check_decode_plan(const at::Tensor& plan, const at::Tensor& q) {
     TORCH_CHECK(plan.device() == q.device(), "ie: plan must be on q's device");
 }
 
+// plan_rows of the planned launch: decode_plan's lists have exactly the launch's entries.
+int64_t decode_plan_rows(const at::Tensor& plan, const DecodeCall& d) {
+    const int32_t units = ie_decode_attention_units(d.B, d.hq, (int32_t)d.c.num_kv_heads);
+    const int64_t rows = plan.size(0);
+    return rows == ie_decode_attention_grid(d.B, units) ? rows + IE_PLAN_LAUNCH_UNITS : rows;
+}
+
 // The kept decode workspace a call uses: calls of up to 1024 sequences and 128 query heads
 // share one (their count regions coincide), every larger shape has one of its own.
 int32_t decode_ws_kind(const DecodeCall& d) {
@@ -476,9 +483,9 @@ void decode_attention(const at::Tensor& q, const at::Tensor& k_cache, const at::
         check_decode_plan(*plan, q);
         ok(ie_decode_attention_planned(bf(q), q.stride(0), q.stride(1), d.B, d.hq, &d.c,
                                        i32(cached_lens), i32(slot_ids), i32(num_decoding),
-                                       i32(*plan), plan->size(0), (float)scale, bfm(out),
-                                       out.stride(0), out.stride(1), ws.data_ptr(), d.ws_bytes,
-                                       stream_of(q)),
+                                       i32(*plan), decode_plan_rows(*plan, d), (float)scale,
+                                       bfm(out), out.stride(0), out.stride(1), ws.data_ptr(),
+                                       d.ws_bytes, stream_of(q)),
            "decode_attention");
         return;
     }
@@ -523,9 +530,9 @@ void decode_attention_rope(const at::Tensor& q, const at::Tensor& k, const at::T
                bf(q), q.stride(0), q.stride(1), bf(k), k.stride(0), k.stride(1), bf(v),
                v.stride(0), v.stride(1), bf(q_norm_weight), bf(k_norm_weight), bf(cos),
                cos.stride(0), bf(sin), sin.stride(0), (float)eps, d.B, d.hq, &d.c,
-               i32(cached_lens), i32(slot_ids), i32(num_decoding), i32(*plan), plan->size(0),
-               (float)scale, bfm(out), out.stride(0), out.stride(1), ws.data_ptr(), d.ws_bytes,
-               stream_of(q)),
+               i32(cached_lens), i32(slot_ids), i32(num_decoding), i32(*plan),
+               decode_plan_rows(*plan, d), (float)scale, bfm(out), out.stride(0), out.stride(1),
+               ws.data_ptr(), d.ws_bytes, stream_of(q)),
            "decode_attention_rope");
         return;
     }
@@ -577,8 +584,8 @@ at::Tensor decode_plan(const at::Tensor& cached_lens, const at::Tensor& num_deco
     TORCH_CHECK(num_kv_heads > 0 && num_q_heads > 0 && num_q_heads % num_kv_heads == 0 &&
                     num_q_heads / num_kv_heads <= 16,
                 "ie: num_q_heads must be num_kv_heads times a GQA ratio of 1 to 16");
-    const int32_t units =
-        (int32_t)(num_kv_heads * ((num_q_heads / num_kv_heads + 1) / 2));
+    const int32_t units = ie_decode_attention_units((int32_t)batch, (int32_t)num_q_heads,
+                                                    (int32_t)num_kv_heads);
     const int32_t grid = ie_decode_attention_grid((int32_t)batch, units);
     at::Tensor rows = at::empty({std::max(grid, 1), 4}, cached_lens.options());
     ok(ie_decode_attention_plan(i32(cached_lens), i32(num_decoding), (int32_t)batch, units,
@@ -640,8 +647,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> decode_step_prologue(
     const c10::DeviceGuard guard(cached_lens.device());
     const int64_t B = ids.numel(), D = embed.size(1), H = inv_freq.size(0);
     TORCH_CHECK(cached_lens.size(0) >= B, "ie: cached_lens too short");
-    const int32_t units =
-        (int32_t)(num_kv_heads * ((num_q_heads / num_kv_heads + 1) / 2));
+    const int32_t units = ie_decode_attention_units((int32_t)B, (int32_t)num_q_heads,
+                                                    (int32_t)num_kv_heads);
     const int32_t grid = ie_decode_attention_grid((int32_t)B, units);
     at::Tensor rows = at::empty({std::max(grid, 1), 4}, cached_lens.options());
     auto bopt = embed.options();

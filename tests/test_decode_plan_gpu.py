@@ -100,6 +100,31 @@ def test_planned_decode_other_ratios(ie, workloads, dev, hq, hkv):
     assert torch.equal(outs[0], outs[1]), f"{hq}/{hkv}"
 
 
+@pytest.mark.parametrize("hq,hkv,batch", [(16, 8, 6), (8, 8, 6), (32, 8, 6), (40, 8, 6), (64, 8, 70),
+                                          (64, 4, 6), (16, 1, 6), (40, 8, 300)])
+def test_planned_launch_reads_its_list(ie, workloads, dev, hq, hkv, batch):
+    """At every ratio the planned launch takes its entries from the list: with the entry of a
+    sequence of one piece marked idle in a copy, that sequence alone stays unwritten."""
+    ctx = [300, 2000, 77, 4096, 1, 1500] + [60] * (batch - 6)
+    wl = workloads.decode_workload(ctx, seed=62, hq=hq, hkv=hkv).to(dev)
+    plan = ie.decode_plan(wl.cached_lens, wl.num_decoding, batch, hq, hkv)
+    rows = plan.tolist()
+    w = next(i for i, r in enumerate(rows) if r[0] == 2 and r[2] == 1)
+    idle = plan.clone()
+    idle[w, 2] = 0
+    outs = []
+    for p in (None, plan, idle):
+        o = torch.full_like(wl.q, 7.0)
+        ie.decode_attention(wl.q, wl.cache, wl.cached_lens, wl.slot_ids, wl.num_decoding, SCALE,
+                            out=o, plan=p)
+        outs.append(o)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert (outs[2][2] == 7.0).all()
+    keep = torch.arange(batch, device=dev) != 2
+    assert torch.equal(outs[2][keep], outs[0][keep])
+
+
 def test_one_plan_two_layers_in_graph(ie, dev):
     """A graph computing the plan once and running two layers' fused decode launches from it,
     replayed three times with new lengths (every sequence one token longer) and new q rows in
