@@ -644,13 +644,12 @@ decode_attention_kernel(DecodeArgs a) {
         float mx = -INFINITY;
 #pragma unroll
         for (int v = 0; v < CB; ++v) mx = fmaxf(mx, pm[v]);
-        for (int s0 = CB; s0 < needed; s0 += CB) {
-            float mv[CB];
-#pragma unroll
-            for (int v = 0; v < CB; ++v)
-                mv[v] = s0 + v < needed ? ld_dev(a.part_m + row0 + s0 + v) : -INFINITY;
-#pragma unroll
-            for (int v = 0; v < CB; ++v) mx = fmaxf(mx, mv[v]);
+        // the other maxima, one per lane of the head's 32 (a batch of CB at a time, as the partials:
+        // 64 pieces of 64/4 heads, B=1 ctx 8190, 20.6 us against 19.1)
+        if (needed > CB) {
+            for (int s = CB + (q & 31); s < needed; s += 32)
+                mx = fmaxf(mx, ld_dev(a.part_m + row0 + s));
+            mx = max_xor16(max16(mx));
         }
         f32x4_t num = {0.f, 0.f, 0.f, 0.f};
         float den = 0.0f;
