@@ -848,6 +848,25 @@ TORCH_LIBRARY_IMPL(ie, Autograd, m) {
     m.impl("decode_attention_rope_new", torch::CppFunction::makeFallthrough());
 }
 
+// For tracing (fake and meta tensors): their output's shape and type.
+at::Tensor decode_attention_new_meta(const at::Tensor& q, const at::Tensor&, const at::Tensor&,
+                                     const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                                     const at::Tensor&, const at::Tensor&, const at::Tensor&, double,
+                                     const c10::optional<at::Tensor>&) {
+    return at::empty_symint(q.sym_sizes(), q.options());
+}
+at::Tensor decode_attention_rope_new_meta(
+    const at::Tensor& q, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+    const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+    const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+    double, double, const c10::optional<at::Tensor>&) {
+    return at::empty_symint(q.sym_sizes(), q.options());
+}
+TORCH_LIBRARY_IMPL(ie, Meta, m) {
+    m.impl("decode_attention_new", &decode_attention_new_meta);
+    m.impl("decode_attention_rope_new", &decode_attention_rope_new_meta);
+}
+
 TORCH_LIBRARY_IMPL(ie, CUDA, m) {
     m.impl("quantize_kv_prefill", &quantize_kv_prefill);
     m.impl("fused_rope_kv_decode", &fused_rope_kv_decode);
