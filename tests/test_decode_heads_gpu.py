@@ -1,5 +1,5 @@
 """The decode kernel's tiles at their edges: a wave's block holds 32 tokens, a workgroup round 32 per
-wave (4-, 2- and one-wave workgroups by batch), the 16 columns of a tile hold a KV head's query
+wave (8-, 4-, 2- and one-wave workgroups by batch and heads), the 16 columns of a tile hold a KV head's query
 heads. Sequence lengths around those sizes at odd and full ratios, workgroups of every width, the
 few-KV-head layouts whose entries are cut to the workspace, `out` rows that take no 8-byte store, and
 V scales that leave the fp16 window mid-sequence; against the oracle with the bf16 tolerance."""
@@ -82,11 +82,23 @@ def test_v_scales_that_move(ie, workloads, dev, hq, hkv):
     assert_attn_close(got / scale, ref / scale, "moving V scales", rel=False)
 
 
-def test_fused_form_many_heads_one_wave_workgroups(ie, dev):
-    """decode_attention_rope where q's rows lie over the second stage (ratio 16, one wave per
-    workgroup): the same outputs as fused_rope_kv_decode then decode_attention, bit for bit in the
-    cache, within the tolerance in the output (the new token enters from registers)."""
-    hq, hkv, B, L = 64, 4, 520, 400
+@pytest.mark.parametrize("hq,hkv,B,waves", [
+    (64, 4, 300, 1), (128, 8, 140, 1),  # q's rows over the second stage: one wave, over 8 heads
+    (64, 8, 150, 1), (16, 8, 140, 1),   # one wave, q's rows beside the stages
+    (64, 4, 520, 2), (64, 8, 100, 2),
+    (64, 8, 12, 4), (40, 8, 5, 4),
+    (64, 4, 20, 8), (16, 1, 4, 8), (12, 4, 30, 8)])
+def test_fused_form_in_every_width(ie, native, dev, hq, hkv, B, waves):
+    """decode_attention_rope in workgroups of every number of waves: the same cache, bit for bit, as
+    fused_rope_kv_decode then decode_attention, and the same output within the tolerance (there q
+    comes from memory and the new token from the cache). Lengths at which every wave has blocks of
+    both its stages."""
+    L = 400 if waves <= 2 else 6000
+    lib = native.cabi()
+    units = lib.ie_decode_attention_units(B, hq, hkv)
+    width = {lib.ie_decode_attention_max_splits(units) // w: w for w in (1, 2, 4)}
+    named = min(8, width.get(lib.ie_decode_attention_target(B, units), 0) * units // hkv)
+    assert named == waves, f"the launch has {named}-wave workgroups"
     g = torch.Generator().manual_seed(75)
     qkv = torch.randn(B, (hq + 2 * hkv) * 128, generator=g).bfloat16().to(dev)
     q, k, v = (x.view(B, -1, 128) for x in qkv.split([hq * 128, hkv * 128, hkv * 128], -1))
