@@ -2,7 +2,8 @@
 leaves the busiest CU fewer columns) against the reordered weight's launches, whose result bits at an
 even width are those of the separate-tile row-major form: the same bits, at row counts around the
 16-row tiles, plain and with the RMSNorm inside, for column counts that do and do not divide into
-24-column workgroups. And the 8-row form through LDS stages against 16-row tiles."""
+24-column workgroups. And the 8-row form through LDS stages: against float64, and bit for bit against
+the form without them (which weights of more row blocks than CUs take)."""
 
 import pytest
 import torch
@@ -34,6 +35,42 @@ def test_row_pairs_bits(ie, dev, M, N, K, nt):
     b = ops.skinny_matmul_norm(x, sw, 2 * nt, True, 1e-6, True, False)
     torch.cuda.synchronize()
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(6144, 1024), (2304, 512), (9216, 2048), (24576, 256)])
+def test_row_pairs_bits_at_other_widths(ie, dev, M, N, K):
+    """Widths where 24-column workgroups replace 32-column ones (n_tiles 2)."""
+    say(f"gate/up {N}x{K} M={M}")
+    x, w = _mats(dev, M, N, K, 93)
+    a = ie.skinny_matmul_silu_mul(x, w, 2)
+    b = ie.skinny_matmul_silu_mul(x, ie.swizzle_weight(w, 4, gate_up=True), 4, swizzled=True)
+    torch.cuda.synchronize()
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("K", [512, 2048, 6144])
+def test_eight_row_stages_bits(ie, dev, M, K):
+    """The first rows of a weight alone (one 8-row block per CU at most: through the stages) and as part
+    of one of twice as many blocks as CUs (without): the same bits, plain, with the RMSNorm and with the
+    residual add; x rows of a wider buffer."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    few, many = 8 * cus, 16 * cus
+    say(f"8-row tiles M={M} K={K}")
+    x, w = _mats(dev, M, many, K, 94)
+    wide = torch.randn(M, K + 64, device=dev).bfloat16()
+    wide[:, :K] = x
+    x = wide[:, :K]
+    ops = torch.ops.ie
+    for f in (lambda w, n: ie.skinny_matmul(x, w, 0),
+              lambda w, n: ops.skinny_matmul_norm(x, w, 0, False, 1e-6, False, False),
+              lambda w, n: ops.skinny_matmul_residual_(x, w, 0, res[:, :n].contiguous(), False,
+                                                       False)):
+        res = torch.randn(M, many, device=dev).bfloat16()
+        a, b = f(w[:few], few), f(w, many)
+        torch.cuda.synchronize()
+        assert torch.equal(a.view(torch.int16), b[:, :few].contiguous().view(torch.int16))
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 40, 64])
