@@ -66,16 +66,16 @@ def test_workspace_size_formula(native):
     lib.ie_decode_attention_grid.restype = ctypes.c_int32
     prev = 0
     for B in (1, 64, 65, 96, 128, 129, 256, 257, 300, 1024):
-        # the target grows with the batch (8-, 4- then 2-wave workgroups) and holds it while
+        # the target grows with the batch (4-, 2- then one-wave workgroups) and holds it while
         # any launch shape can
         target = lib.ie_decode_attention_target(ctypes.c_int32(B), ctypes.c_int32(8))
         assert prev <= target <= t_max and (B <= target or target == t_max)
         prev = target
         grid = lib.ie_decode_attention_grid(ctypes.c_int32(B), ctypes.c_int32(8))
         assert grid == (target if B <= target else target + B)
-        # counts: one per sequence and query head (the most any GQA ratio uses), for at least
-        # 1024 sequences and 128 heads; partials: one per query head and work entry of the
-        # largest grid (cdiv(Hq, 2) units: GQA 2)
+        # counts: one per sequence and query head (a launch uses one per sequence and KV head), for
+        # at least 1024 sequences and 128 heads; partials: one per query head and work entry of the
+        # grid of 8 units (cdiv(Hq, 2), GQA 2), which holds what any other ratio's launch is cut for
         counts = -(-(max(B, 1024) * 128) * 4 // 256) * 256
         assert lib.ie_decode_attention_workspace_size(B, 16, 128) == counts + 16 * grid * 130 * 4
 

@@ -107,7 +107,7 @@ def sampled_check(ie, workloads, dev, ctx, pick, seed, what, **kw):
 @pytest.mark.parametrize("B,ctx", [(64, 4096), (16, 4096), (256, 1024), (256, 4096)])
 def test_decode_config3_sampled(ie, workloads, dev, B, ctx):
     """BASELINE config 3 points at full size, generated on the GPU (B=64 ctx=4096 is the
-    headline, 8-wave workgroups; B=256 runs 2-wave workgroups, whose per-head target of 256
+    headline, 4-wave workgroups; B=256 runs one-wave workgroups, whose per-head target of 256
     holds the batch): 8 sampled sequences checked against the oracle."""
     say(f"decode config 3 B={B} ctx={ctx} (sampled)")
     pick = sorted({0, 1, B // 4, B // 2 - 1, B // 2, 3 * B // 4, B - 2, B - 1})
@@ -115,13 +115,13 @@ def test_decode_config3_sampled(ie, workloads, dev, B, ctx):
 
 
 @pytest.mark.parametrize("B,nd,lo,hi,seed", [
-    (200, 170, 1, 3000, 31),  # 2-wave workgroups (target 256 on 256 CUs), fitted pieces
+    (200, 170, 1, 3000, 31),  # one-wave workgroups (target 256 on 256 CUs), fitted pieces
     (300, 299, 1, 600, 32),   # above every target: the reference's TARGET + B grid
-    (65, 65, 2000, 9000, 33),  # one past the 8-wave target: 4-wave workgroups, several splits
+    (65, 65, 2000, 9000, 33),  # one past the 4-wave target: 2-wave workgroups, several splits
 ])
 def test_decode_ragged_large_batch(ie, workloads, dev, B, nd, lo, hi, seed):
-    """Batches above the 8-wave workgroups' per-head target (64 on 256 CUs) with
-    num_decoding < B: 4- and 2-wave workgroups with fitted pieces, and above every target the
+    """Batches above the 4-wave workgroups' per-head target (64 on 256 CUs) with
+    num_decoding < B: 2- and one-wave workgroups with fitted pieces, and above every target the
     reference's unfitted piece rule and TARGET + B grid (kernels.py:294-314); every decoding row
     against the oracle and the rows past num_decoding untouched."""
     ctx = [int(x) for x in np.random.default_rng(seed).integers(lo, hi + 1, B)]
@@ -138,7 +138,7 @@ def test_decode_ragged_large_batch(ie, workloads, dev, B, nd, lo, hi, seed):
 
 
 def test_decode_long_and_short_mix_above_target(ie, workloads, dev):
-    """96 sequences, 6 of them 30-60K tokens long (4-wave workgroups): the long ones split into
+    """96 sequences, 6 of them 30-60K tokens long (2-wave workgroups): the long ones split into
     many pieces, merged by their last piece."""
     rng = np.random.default_rng(41)
     ctx = [int(x) for x in rng.integers(100, 500, 90)] + [int(x) for x in

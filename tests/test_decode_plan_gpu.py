@@ -1,7 +1,7 @@
 """decode_attention / decode_attention_rope with the step's work list computed once (decode_plan,
 then ie_decode_attention_planned / ie_decode_attention_rope_planned): outputs and cache writes
 bit for bit equal to the launches that derive the list from cached_lens themselves, over the
-launch shapes (8-, 4- and 2-wave workgroups, one piece per sequence, split sequences, padding
+launch shapes (4-, 2- and one-wave workgroups, one piece per sequence, split sequences, padding
 rows past num_decoding), other GQA ratios, one plan serving two layers, and a replayed graph
 whose inputs change between replays. The self-scheduling launches are the ones the oracle tests
 pin (test_decode_gpu.py, test_decode_rope_gpu.py); one case here is also checked against the
@@ -22,8 +22,8 @@ SHAPES = [
     ([int(x) for x in np.random.default_rng(5).integers(128, 4096, 32)], 32),  # config 5
     ([4096] * 63 + [1], 64),                    # one piece per sequence
     ([1, 2, 130, 3000, 7, 257, 64, 65, 900, 4000, 33, 512, 129], 11),  # padding rows
-    ([int(x) for x in np.random.default_rng(7).integers(1, 1500, 100)], 100),  # 4 waves
-    ([int(x) for x in np.random.default_rng(6).integers(1, 600, 300)], 297),   # 2 waves
+    ([int(x) for x in np.random.default_rng(7).integers(1, 1500, 100)], 100),  # 2 waves
+    ([int(x) for x in np.random.default_rng(6).integers(1, 600, 300)], 297),   # one wave
 ]
 
 

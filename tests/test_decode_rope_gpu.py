@@ -49,8 +49,8 @@ def _case(ie, lens, nd, seed, max_len):
     ([1, 2, 130, 3000, 7, 257, 64, 65, 900, 4000, 33, 512, 129], 11),  # padding rows after 11
     ([int(x) for x in np.random.default_rng(5).integers(128, 4096, 32)], 32),  # config 5
     ([4096] * 63 + [1], 64),                             # one piece per sequence, full target
-    ([int(x) for x in np.random.default_rng(6).integers(1, 600, 300)], 297),  # 2-wave launch
-    ([int(x) for x in np.random.default_rng(7).integers(1, 1500, 100)], 100),  # 4-wave launch
+    ([int(x) for x in np.random.default_rng(6).integers(1, 600, 300)], 297),  # one-wave launch
+    ([int(x) for x in np.random.default_rng(7).integers(1, 1500, 100)], 100),  # 2-wave launch
 ])
 def test_decode_attention_rope(ie, dev, lens, nd):
     say(f"decode_attention_rope B={len(lens)} nd={nd} max ctx {max(lens)}")
@@ -59,7 +59,7 @@ def test_decode_attention_rope(ie, dev, lens, nd):
 
 @pytest.mark.parametrize("seed", range(4))
 def test_decode_attention_rope_random(ie, dev, seed):
-    """Seeded random batches across the three launch shapes (8-, 4- and 2-wave workgroups):
+    """Seeded random batches across the three launch shapes (4-, 2- and one-wave workgroups):
     1-300 sequences of 1-1,500 tokens, padding rows after num_decoding."""
     rng = np.random.default_rng(200 + seed)
     B = int((rng.integers(1, 65), rng.integers(65, 129), rng.integers(129, 301))[seed % 3])
