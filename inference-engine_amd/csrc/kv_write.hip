@@ -807,7 +807,12 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Row groups per wave of norm_rope_rows_kernel: one while the step is small (latency: 64 tokens of
 // 16 + 8 heads 2.5 us, against 4.2 with six; 1,054 tokens 5.2 against 6.3), six or three from about
 // 4,096 such tokens (the token's cos and sin and the weights are read once per wave: 12,288 tokens
-// 29.6 us against 34.6 with one).
+// 29.6 us against 34.6 with one). Six where they divide the groups or number 12 and more, else three.
+// Other head counts at 98,400 / 200,000 / 400,000 rows, us with 1, 3 and 6 groups: 8 + 4 heads 13.8,
+// 13.4, 16.7 / 24.4, 22.7, 28.2 / 43.0, 37.6, 48.1; 32 + 8 13.6, 14.3, 13.9 / 23.3, 23.9, 22.0 / 44.3,
+// 40.9, 37.7; 40 + 8 14.0, 13.6, 14.0 / 24.2, 22.8, 22.0 / 43.6, 38.0, 36.8; 64 + 4 13.9, 13.8, 14.2 /
+// 24.0, 22.9, 22.5 / 44.3, 39.0, 37.2. At 60,000 rows one is ahead at every head count (9.5 against
+// 10 to 12).
 static int nr_groups(int64_t tokens, int rows) {
     const int groups = (rows + 3) / 4;
     if (tokens * rows < 4096 * 24 || groups < 3) return 1;
@@ -912,7 +917,9 @@ extern "C" hipError_t ie_fused_norm_rope_prefill(
                             cos_stride_tok | sin_stride_tok | q_out_stride_tok |
                             q_out_stride_head | k_out_stride_tok | k_out_stride_head;
     // (a few tokens of at most four rows finish sooner with a wave per row: 16 tokens of 2 + 1 heads
-    // 2.3 against 2.4 us, 1,054 tokens 3.1 against 2.8)
+    // 2.28 against 2.38 us, 512 2.49 against 2.49, 1,054 3.03 against 2.79; 1 + 1 heads 2.18 against
+    // 2.31, 2.46 against 2.47 and 2.93 against 2.75; 3 + 1 2.29 against 2.40, 2.52 against 2.50 and
+    // 3.12 against 2.85)
     if (!(rows <= 4 && num_tokens <= 512) && strides % 8 == 0 && aligned16(q) && aligned16(k) &&
         aligned16(q_norm_weight) && aligned16(k_norm_weight) && aligned16(cos) && aligned16(sin) &&
         aligned16(q_out) && aligned16(k_out)) {

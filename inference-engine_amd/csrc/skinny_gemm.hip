@@ -83,8 +83,8 @@ constexpr int SG_MAX_TILES = 6;  // weight + x tiles, at most (LDS: 8 waves x 16
 // down projection), rows past M not written.
 // RPAIR (with GLU, row-major): the paired tiles of SWZ's gate/up order read from the row-major
 // weight (half a tile's rows from the gate part, half from the up part), 8 NT columns per workgroup.
-// DMA (with HALF): the batches go straight to LDS (dma16), three or four of them in flight per wave
-// with no registers held and no store to LDS; the same fragments in the same order.
+// DMA (with HALF): the batches go straight to LDS (dma16), two (from 33 rows on) to four of them in
+// flight per wave with no registers held and no store to LDS; the same fragments in the same order.
 // AMAX (with LOOP and XREG: the LM head): also the greedy token of every row, the first column
 // of the largest bf16 output (sample's greedy rule at tau = 0: larger value, then smaller index;
 // NaN never chosen): each lane keeps its best over its blocks, each workgroup folds its lanes'
@@ -717,7 +717,10 @@ void sg_glu_mt(int mt, int n_tiles, dim3 grid, hipStream_t s, const SgCall& c) {
 // CU then has fewer columns to do than in 16 n_tiles-column workgroups, every CU working (6,144
 // columns: 256 workgroups of 24, against 192 of 32 or 384 of 16). The same bits.
 // Measured at [12288, 2048], 1 / 16 / 32 / 48 rows: 12.5 / 12.8 / 14.3 / 18.6 -> 11.5 / 11.5 / 12.7 /
-// 14.4 us.
+// 14.4 us, [9216, 2048] 10.4 / 10.8 / 12.2 / 17.4 -> 9.4 / 9.6 / 10.9 / 12.6. Against 32-column
+// workgroups alone (16-column ones have no more a CU than 24), 1 / 16 / 32 rows: [2304, 2048] 8.5 / 9.0 /
+// 10.6 -> 7.3 / 7.8 / 9.4, [6144, 2048] 9.3 / 9.9 / 11.3 -> 8.1 / 8.7 / 10.1, [19200, 2560] 26.0 / 27.6
+// / 31.1 -> 21.6 / 22.7 / 27.1, [24576, 4096] 38.7 / 41.2 / 41.6 -> 34.0 / 34.5 / 36.9.
 bool sg_row_pairs(int cols, int n_tiles, int mt) {
     const int cus = device_cu_count();
     auto most = [&](int per) { return (cols / per + cus - 1) / cus * per; };
