@@ -787,7 +787,9 @@ static Layout workspace_size_layout(int batch, int hq) {
 // hold it without (16/16 heads B=129-256 on 256 CUs: 257-384 entries, 256 reserved): the entries
 // reserved, then.
 static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes = SIZE_MAX) {
-    const Layout S = workspace_size_layout(batch, hq), own = workspace_layout(batch, hq, hkv);
+    const Layout own = workspace_layout(batch, hq, hkv);
+    if (hq == 2 * hkv) return own;  // one of the two that the workspace is made for
+    const Layout S = workspace_size_layout(batch, hq);
     // the widest workgroups of which every entry is resident (one-wave ones where none is): 12/4
     // heads B=300 have 341 entries a head, 5 rounds of 8-wave workgroups
     auto resident_waves = [&](int entries) {
@@ -795,7 +797,7 @@ static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes = SIZE_MA
         while (w > 1 && decode_target(hkv, w) < entries) w /= 2;
         return w;
     };
-    if (hq <= 2 * hkv)
+    if (hq < 2 * hkv)
         return own.bytes <= S.bytes ? own : layout_of(batch, hq, resident_waves(S.nwork), S.target);
     const size_t room = std::min(S.bytes, max_bytes), row = (DA_D + 2) * sizeof(float);
     const int fit = room > S.acc_off ? (int)((room - S.acc_off) / (hq * row)) : 0;
@@ -812,6 +814,7 @@ static Layout call_layout(int batch, int hq, int hkv, size_t max_bytes = SIZE_MA
 // The num_units whose work list has a call's entries (a list depends on the batch and the target
 // alone), or 0: none of the unit counts that a layout comes from gives that target.
 static int list_units(int batch, int hq, int hkv) {
+    if (hq == 2 * hkv) return hkv;
     const int target = call_layout(batch, hq, hkv).target, pairs = std::max(1, (hq + 1) / 2);
     for (int u : {hkv, 2 * hkv, 4 * hkv, 8 * hkv, std::min(8, pairs), pairs})
         if (workspace_layout(batch, hq, u).target == target) return u;
@@ -825,7 +828,7 @@ using namespace ie;
 extern "C" size_t ie_decode_attention_workspace_counts_bytes(int32_t batch,
                                                              int32_t num_q_heads) {
     if (num_q_heads <= 0) return 0;
-    return workspace_size_layout(batch, num_q_heads).acc_off;
+    return layout_of(std::max(batch, 0), num_q_heads, 1, 1).acc_off;  // whatever the entries
 }
 
 extern "C" int32_t ie_decode_attention_max_splits(int32_t num_units) {
