@@ -92,25 +92,19 @@ int decode_units(int hq, int hkv) { return hkv * ((hq / std::max(1, hkv) + 1) / 
 __device__ int decode_piece(const int32_t* __restrict__ cached_lens, int nd, int target, int n0) {
     const int lane = threadIdx.x & 63;
     auto n_of = [&](int b0) { return b0 == 0 ? n0 : (b0 + lane < nd ? cached_lens[b0 + lane] + 1 : 0); };
-    // summed per lane first, so that the loads of several 64 sequences are in flight together and the
-    // wave adds up once
     int total = 0, longest = 0;
-#pragma unroll 4
     for (int b0 = 0; b0 < nd; b0 += 64) {
         const int n = n_of(b0);
-        total += n;
-        longest = max(longest, n);
+        total += wave_sum_i(n);
+        longest = max(longest, (int)wave_max((float)n));
     }
-    total = wave_sum_i(total);
-    longest = (int)wave_max((float)longest);
     const int k0 = max(1, cdiv_i(cdiv_i(total, target), DA_MIN_PIECE));
     if (nd > target) return k0 * DA_MIN_PIECE;
     auto pieces = [&](int k) {
         const Divisor p = divisor(k * DA_MIN_PIECE);
         int c = 0;
-#pragma unroll 4
-        for (int b0 = 0; b0 < nd; b0 += 64) c += div_ceil(n_of(b0), p);
-        return wave_sum_i(c);
+        for (int b0 = 0; b0 < nd; b0 += 64) c += wave_sum_i(div_ceil(n_of(b0), p));
+        return c;
     };
     int lo = k0, hi = max(k0, cdiv_i(longest, DA_MIN_PIECE));  // pieces(hi) <= nd <= target
     while (lo < hi) {
